@@ -76,7 +76,7 @@ class DeviceModel:
                   lm_type: int = EL.Q8_0, embed_type: int = EL.BF16, std: float = 0.02) -> "DeviceModel":
         H.init()
         m = cls(cfg, seed, frozenset(q8))
-        biggest = max(cfg.V * cfg.D, cfg.F * cfg.D)
+        biggest = max(cfg.V, cfg.F, cfg.D) * cfg.D  # embedding and head, feed-forward, q and o
         scratch = H.DeviceArray((biggest,), np.float32)
         tid = 0
 
