@@ -7,6 +7,7 @@
 // product uses the 8-way partial sums of kern::dot_f32 (src/kernels.cpp:27-43), softmax subtracts
 // the max, uses float exp and a double sum (:77-92), and each output dimension accumulates p * v
 // over positions in order (:168-172).
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -1048,148 +1049,158 @@ __global__ __launch_bounds__(kAttnThreads) void prefill_attention_kernel(Prefill
                 a.a.ctx + static_cast<long>(r) * a.a.ldq + h * hd, nullptr);
 }
 
-// Prefill, step 2 for long prompts (hd = 64, at most 8 query heads per KV head): workgroup (x, g)
-// takes kPfRows consecutive rows of one sequence and KV group g, so each staged 64-position chunk of
-// K / V serves every (row, head) pair of the block instead of one.  Thread t owns pair t % 128
-// (row t % 128 / hpg, head t % 128 % hpg) with its roped query in registers, and half t / 128 of
-// each chunk's positions.  Scores follow kern::dot_f32's order (src/kernels.cpp:27-43).  Two passes
-// over the chunks: the row's maximum, then e = float exp(s - max), their double sum (each half in
-// position order, then the two halves) and o[d] = sum_t e_t v_t[d] over positions in increasing
-// order (thread: its pair, dimensions 32 (t / 128) ..); out = o * float(1 / sum).  The reference
-// scales each e by 1 / sum before the p.v sum (src/kernels.cpp:77-92,153-174): the results differ
-// by that rounding.  Rows, chunk rows past the block's last position and positions past a row's
-// own take no part (zero K / V rows, e = 0).
-constexpr int kPfRows = 16, kPfChunk = 64, kPfLd = 68, kPfPairs = 128, kPfPsLd = 65;
-constexpr int kPfTileFrom = 128;  // positions per sequence in a launch from which the tiled kernel runs
+// Prefill, step 2 on the matrix cores (hd = 64, up to kPfPairs query heads per KV head): a workgroup
+// takes kPfPairs (row, query head) pairs of one sequence and KV group (consecutive rows, every head
+// of the group), so each 64-position chunk of K / V is staged in LDS once for all of them; wave w
+// owns pairs 16 w .. 16 w + 15.  One pass over the chunks with a running maximum.
+//
+// Everything stays FP32: v_mfma_f32_16x16x4_f32 on the cache's own values (no conversion), lane
+// l = 16 g + m.  S^T = K Q^T puts a pair's scores in its own lanes (D: positions 4 g + r, pair m), and
+// since a product's k slots may hold any four positions, slot g of step r takes position 4 g + r:
+// the exponentials feed O^T += V^T P^T straight from the registers they were computed in.  K and Q
+// columns are taken as dims 16 j + 4 g + s and V's as 4 m + t, so every LDS read is 16 bytes and
+// the lane's outputs are dims 16 g .. 16 g + 15 of its pair.
+//
+// Scores, exponentials and p.v are FP32, the sum of a row's exponentials is double, as in
+// kern::attention_heads (src/kernels.cpp:77-92,153-174); a chunk's p.v is summed on its own and
+// added to the running one, each new maximum rescales the running sums, and 1 / sum is applied at the
+// end.  Scores have two partial sums and p.v one per chunk, so no chain of additions is long.
+// Positions past a row's own take no part (score -inf, V rows past the block's last position zero); a
+// maximum of -inf subtracts 0, so a row whose first chunks are all -inf still sums the rest.
+//
+// Bound by the FP32 matrix rate (151 TFLOP/s for a large library product on this GPU: 109 us for the
+// causal half of 1999 positions x 32 heads): 186 us, 31 us at 510 positions.  The vector-ALU
+// kernel before it, bound by LDS reads of K, took 1362 and 344 us.
+constexpr int kPfPairs = 64, kPfChunk = 64, kPfLd = 68;
+// The kernel runs from 128 positions per sequence, or from 32 workgroups: below that the one
+// workgroup per (head, row) kernel fills more of the GPU.  Four layers, 32 heads over 4 KV heads,
+// us per prefill, rows kernel / this one: 1 x 8 positions (4 workgroups) 254 / 262, 1 x 23 (12)
+// 280 / 283, 1 x 64 (32) 332 / 318, 4 x 23 (48) 434 / 421, 64 x 23 2636 / 2257.
+constexpr int kPfMfmaFrom = 128, kPfMfmaWorkgroups = 32;
 
-size_t prefill_tile_lds_bytes() {
-  return (2 * kPfChunk * kPfLd + kPfPairs * kPfPsLd + 2 * kPfPairs) * sizeof(float) + 2 * kPfPairs * sizeof(double);
-}
-
-__global__ __launch_bounds__(256) void prefill_tile_kernel(PrefillArgs pa) {
-#pragma clang fp contract(off)
+__global__ __launch_bounds__(256) void prefill_mfma_kernel(PrefillArgs pa, int nseq, int cus) {
   const AttnArgs& a = pa.a;
-  extern __shared__ float sm[];
-  float* ks = sm;                                           // [64][kPfLd] K rows of the chunk
-  float* vs = ks + kPfChunk * kPfLd;                        // [64][kPfLd] V rows
-  float* ps = vs + kPfChunk * kPfLd;                        // [128][kPfPsLd] exponentials of the chunk
-  float* mx2 = ps + kPfPairs * kPfPsLd;                     // [2][128] maxima per half
-  double* l2 = reinterpret_cast<double*>(mx2 + 2 * kPfPairs);  // [2][128] sums per half
-  const int nb = (pa.n + kPfRows - 1) / kPfRows;
-  const int b = blockIdx.x / nb, i0 = (blockIdx.x % nb) * kPfRows, g = blockIdx.y, t = threadIdx.x;
-  const int hpg = a.H / a.KV, kvd = a.KV * 64;
-  const int pair = t & (kPfPairs - 1), half = t >> 7;
-  const int il = pair / hpg, hh = pair - il * hpg, i = i0 + il;
-  const bool active = il < kPfRows && i < pa.n;
+  __shared__ float ks[kPfChunk * kPfLd], vs[kPfChunk * kPfLd];
+  const int t = threadIdx.x, wave = t / kWave, lane = t & (kWave - 1), m = lane & 15, g = lane >> 4;
+  const int hpg = a.H / a.KV, kvd = a.KV * 64, rpb = kPfPairs / hpg;
+  const int nb = (pa.n + rpb - 1) / rpb;
+  // Blocks in decreasing order of their positions, every second round over the CUs reversed: workgroups
+  // are dealt to the CUs in order, so each CU's share of the causal triangle comes out even.
+  int id = blockIdx.x;
+  {
+    const int total = nb * nseq * a.KV, r0 = id / cus * cus, r1 = min(r0 + cus, total);
+    if ((id / cus) & 1) id = r0 + r1 - 1 - id;
+  }
+  const int kv = id % a.KV, b = id / a.KV % nseq, i0 = (nb - 1 - id / a.KV / nseq) * rpb;
+  const int pair = 16 * wave + m, il = pair / hpg, hh = pair - il * hpg, i = i0 + il;
+  const bool active = il < rpb && i < pa.n;
   const int pos0 = *a.pos_dev;
-  const int prow = pos0 + i, plast = pos0 + min(i0 + kPfRows, pa.n) - 1;
-  const long r = static_cast<long>(b) * pa.n + i;
-  float q[64];
-  if (active) {
-    const float4* qp = reinterpret_cast<const float4*>(a.q + r * a.ldq + (g * hpg + hh) * 64);
+  const int prow = pos0 + i, pfirst = pos0 + i0, plast = pos0 + min(i0 + rpb, pa.n) - 1;
+  const long row = static_cast<long>(b) * pa.n + (active ? i : i0);
+  f4n q[4];
+  {
+    const float* qp = a.q + row * a.ldq + (kv * hpg + (active ? hh : 0)) * 64 + 4 * g;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const float4 v = qp[k];
-      q[4 * k] = v.x;
-      q[4 * k + 1] = v.y;
-      q[4 * k + 2] = v.z;
-      q[4 * k + 3] = v.w;
-    }
+    for (int j = 0; j < 4; ++j) q[j] = *reinterpret_cast<const f4n*>(qp + 16 * j);
   }
-  const float* kc = a.kcache + static_cast<long>(b) * a.max_seq * kvd + g * 64;
-  const float* vc = a.vcache + static_cast<long>(b) * a.max_seq * kvd + g * 64;
-  auto stage = [&](float* dst, const float* src, int c0) {
-    for (int idx = t; idx < kPfChunk * 16; idx += 256) {
-      const int rr = idx >> 4, cc = idx & 15;
-      float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (c0 + rr <= plast) v = reinterpret_cast<const float4*>(src + static_cast<long>(c0 + rr) * kvd)[cc];
-      reinterpret_cast<float4*>(dst + rr * kPfLd)[cc] = v;
+  const float* kc = a.kcache + static_cast<long>(b) * a.max_seq * kvd + kv * 64;
+  const float* vc = a.vcache + static_cast<long>(b) * a.max_seq * kvd + kv * 64;
+  // thread t stages columns 4 (t % 16) .. of rows t / 16 + 16 u of a chunk
+  f4n kr[4], vr[4];
+  auto fetch = [&](int c0) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int p = c0 + t / 16 + 16 * u;
+      const long o = static_cast<long>(min(p, plast)) * kvd + 4 * (t & 15);
+      kr[u] = *reinterpret_cast<const f4n*>(kc + o);
+      vr[u] = *reinterpret_cast<const f4n*>(vc + o);
+      if (p > plast) vr[u] = f4n{0.0f, 0.0f, 0.0f, 0.0f};
     }
   };
-  auto score = [&](int rr) -> float {
-    const float* kr = ks + rr * kPfLd;
-    float p0 = 0.0f, p1 = 0.0f, p2 = 0.0f, p3 = 0.0f, p4 = 0.0f, p5 = 0.0f, p6 = 0.0f, p7 = 0.0f;
+  f4n o[4];
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      const float4 ka = *reinterpret_cast<const float4*>(kr + 8 * m);
-      const float4 kb = *reinterpret_cast<const float4*>(kr + 8 * m + 4);
-      p0 += q[8 * m] * ka.x;
-      p1 += q[8 * m + 1] * ka.y;
-      p2 += q[8 * m + 2] * ka.z;
-      p3 += q[8 * m + 3] * ka.w;
-      p4 += q[8 * m + 4] * kb.x;
-      p5 += q[8 * m + 5] * kb.y;
-      p6 += q[8 * m + 6] * kb.z;
-      p7 += q[8 * m + 7] * kb.w;
-    }
-    return (((p0 + p1) + (p2 + p3)) + ((p4 + p5) + (p6 + p7))) * a.scale;
-  };
-  const int nchunks = plast / kPfChunk + 1;
-  // pass 1: each row's maximum
-  float m = -INFINITY;
-  for (int c = 0; c < nchunks; ++c) {
-    stage(ks, kc, c * kPfChunk);
-    __syncthreads();
-    if (active) {
-      for (int j = 0; j < 32; ++j) {
-        const int rr = 32 * half + j;
-        if (c * kPfChunk + rr <= prow) m = fmaxf(m, score(rr));
-      }
-    }
-    __syncthreads();
-  }
-  mx2[half * kPfPairs + pair] = m;
-  __syncthreads();
-  const float M = fmaxf(mx2[pair], mx2[kPfPairs + pair]);
-  // pass 2: exponentials, their sum and the unnormalised p.v
+  for (int d = 0; d < 4; ++d) o[d] = f4n{0.0f, 0.0f, 0.0f, 0.0f};
+  // exponentials as 2^(c2 (s - max)), s the unscaled dot product
+  const float c2 = a.scale * 1.44269504088896340736f;
+  float mx = -INFINITY, sub = 0.0f;
   double l = 0.0;
-  float o[32];
+  fetch(0);
+  for (int c0 = 0; c0 <= plast; c0 += kPfChunk) {
 #pragma unroll
-  for (int d = 0; d < 32; ++d) o[d] = 0.0f;
-  for (int c = 0; c < nchunks; ++c) {
-    stage(ks, kc, c * kPfChunk);
-    stage(vs, vc, c * kPfChunk);
-    __syncthreads();
-    for (int j = 0; j < 32; ++j) {
-      const int rr = 32 * half + j;
-      float e = 0.0f;
-      if (active && c * kPfChunk + rr <= prow) {
-        e = expf(score(rr) - M);
-        l += static_cast<double>(e);
-      }
-      ps[pair * kPfPsLd + rr] = e;
+    for (int u = 0; u < 4; ++u) {
+      const int at = (t / 16 + 16 * u) * kPfLd + 4 * (t & 15);
+      *reinterpret_cast<f4n*>(ks + at) = kr[u];
+      *reinterpret_cast<f4n*>(vs + at) = vr[u];
     }
     __syncthreads();
-    if (active) {
-      for (int rr = 0; rr < kPfChunk; ++rr) {
-        const float e = ps[pair * kPfPsLd + rr];
-        const float* vr = vs + rr * kPfLd + 32 * half;
+    if (c0 + kPfChunk <= plast) fetch(c0 + kPfChunk);
+    f4n sc[4];
 #pragma unroll
-        for (int d = 0; d < 32; d += 4) {
-          const float4 v = *reinterpret_cast<const float4*>(vr + d);
-          o[d] += e * v.x;
-          o[d + 1] += e * v.y;
-          o[d + 2] += e * v.z;
-          o[d + 3] += e * v.w;
+    for (int pt = 0; pt < 4; ++pt) {
+      f4n part[2];  // two partial sums of 32 dims each
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        part[h] = f4n{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 2 * h; j < 2 * h + 2; ++j) {
+          const f4n k = *reinterpret_cast<const f4n*>(ks + (16 * pt + m) * kPfLd + 16 * j + 4 * g);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) part[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[s], q[j][s], part[h], 0, 0, 0);
         }
       }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sc[pt][r] = part[0][r] + part[1][r];
     }
+    if (c0 + kPfChunk > pfirst) {  // a chunk that some row of the workgroup does not see whole
+      const int last = prow - c0 - 4 * g;  // position 16 pt + 4 g + r of the chunk takes part when 16 pt + r <= last
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * pt + r > last) sc[pt][r] = -INFINITY;
+    }
+    float cm = -INFINITY;
+#pragma unroll
+    for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) cm = fmaxf(cm, sc[pt][r]);
+    cm = fmaxf(cm, __shfl_xor(cm, 16, kWave));
+    cm = fmaxf(cm, __shfl_xor(cm, 32, kWave));
+    float al = 1.0f;
+    if (__any(cm > mx)) {
+      const float nm = fmaxf(mx, cm);
+      sub = nm == -INFINITY ? 0.0f : nm * c2;
+      al = __builtin_amdgcn_exp2f(fmaf(mx, c2, -sub));
+      l *= static_cast<double>(al);
+      mx = nm;
+    }
+    f4n oc[4];  // the chunk's own p.v
+#pragma unroll
+    for (int d = 0; d < 4; ++d) oc[d] = f4n{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(sc[pt][r], c2, -sub));
+        l += static_cast<double>(e);
+        const f4n v = *reinterpret_cast<const f4n*>(vs + (16 * pt + 4 * g + r) * kPfLd + 4 * m);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) oc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[d], e, oc[d], 0, 0, 0);
+      }
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[d][r] = fmaf(o[d][r], al, oc[d][r]);
     __syncthreads();
   }
-  l2[half * kPfPairs + pair] = l;
-  __syncthreads();
+  l += __shfl_xor(l, 16, kWave);
+  l += __shfl_xor(l, 32, kWave);
   if (!active) return;
-  const float inv = static_cast<float>(1.0 / (l2[pair] + l2[kPfPairs + pair]));
-  float* out = a.ctx + r * a.ldq + (g * hpg + hh) * 64 + 32 * half;
+  const float inv = static_cast<float>(1.0 / l);
+  float* out = a.ctx + row * a.ldq + (kv * hpg + hh) * 64 + 16 * g;
 #pragma unroll
-  for (int d = 0; d < 32; d += 4) {
-    float4 v;
-    v.x = o[d] * inv;
-    v.y = o[d + 1] * inv;
-    v.z = o[d + 2] * inv;
-    v.w = o[d + 3] * inv;
-    reinterpret_cast<float4*>(out + d)[0] = v;
-  }
+  for (int r = 0; r < 4; ++r)
+    *reinterpret_cast<f4n*>(out + 4 * r) = f4n{o[0][r] * inv, o[1][r] * inv, o[2][r] * inv, o[3][r] * inv};
 }
 
 // x[r] = row hist[b][*pos_dev + i] of the embedding table for every prefill row r = (b, i).
@@ -1279,19 +1290,19 @@ size_t attention_lds_bytes(int hd, int max_seq) {
 int launch_prefill_attention(const PrefillArgs& a, int rows, hipStream_t s) {
   hipLaunchKernelGGL(rope_store_kernel, dim3(rows), dim3(kAttnThreads), 0, s, a);
   EFH_HIP(hipGetLastError());
-  // long prompts (a launch of kPfTileFrom or more positions per sequence): the tiled kernel
+  // long or many prompts: the matrix-core kernel (kPfMfmaFrom)
   const int hpg = a.a.KV > 0 ? a.a.H / a.a.KV : 0;
   const char* forced = std::getenv("EF_HIP_PREFILL_ATTENTION");
-  const bool tiled_ok = a.a.hd == 64 && a.a.H % a.a.KV == 0 && hpg >= 1 && hpg * kPfRows <= kPfPairs &&
-                        a.a.ldq % 4 == 0;
+  const bool tiled_ok = a.a.hd == 64 && a.a.H % a.a.KV == 0 && hpg >= 1 && hpg <= kPfPairs && a.a.ldq % 4 == 0;
   // EF_HIP_PREFILL_ATTENTION=tiled / rows forces either kernel (tests)
   const bool force_rows = forced != nullptr && std::strcmp(forced, "rows") == 0;
   const bool force_tiled = forced != nullptr && std::strcmp(forced, "tiled") == 0;
-  if (tiled_ok && !force_rows && (force_tiled || a.n >= kPfTileFrom)) {
+  const int rpb = tiled_ok ? kPfPairs / hpg : 1, nb = (a.n + rpb - 1) / rpb, nseq = rows / a.n;
+  const bool enough = a.n >= kPfMfmaFrom || static_cast<long>(nseq) * nb * a.a.KV >= kPfMfmaWorkgroups;
+  if (tiled_ok && !force_rows && (force_tiled || enough)) {
     EFH_CHECK(rows % a.n == 0, "prefill attention: rows must be sequences x positions");
-    const int nb = (a.n + kPfRows - 1) / kPfRows;
-    hipLaunchKernelGGL(prefill_tile_kernel, dim3((rows / a.n) * nb, a.a.KV), dim3(256), prefill_tile_lds_bytes(), s,
-                       a);
+    hipLaunchKernelGGL(prefill_mfma_kernel, dim3(static_cast<unsigned>(nseq) * nb * a.a.KV), dim3(256), 0, s, a, nseq,
+                       std::max(1, ctx().cu_count));
     EFH_HIP(hipGetLastError());
     return EF_HIP_OK;
   }

@@ -120,3 +120,28 @@ def test_tiled_prefill_attention_matches_rows_kernel_and_oracle(hip, monkeypatch
         want = ot.forward(int(prompts[0][p]), p, compute_logits=p == n - 1)
     assert _err(got["tiled"][0][0], want) < 1e-4
     ot.close()
+
+
+@pytest.mark.parametrize("H,KV,B,n,rows", [
+    (1, 1, 1, 64, 0),     # one head: 64 rows per workgroup, one exact chunk
+    (3, 1, 2, 65, 0),     # 21 rows x 3 heads (63 of 64 pairs), a one-position second chunk
+    (16, 1, 1, 127, 60),  # 4 rows per workgroup, launches of 60, 60 and 7 positions
+    (8, 4, 3, 1, 0),      # one position per sequence
+])
+def test_matrix_core_prefill_attention_edges(hip, monkeypatch, H, KV, B, n, rows):
+    """The matrix-core prefill attention against the per-(head, row) kernel at the edges of its
+    tiles (pairs, 64-position chunks, a launch that starts past position 0): last logits within 1e-5
+    relative (FP32 sums in another order), as the tiled test above."""
+    cfg = Config(D=64 * H, F=256, H=H, KV=KV, hd=64, V=256, L=2, max_pos=256)
+    if rows:
+        monkeypatch.setenv("EF_HIP_PREFILL_ROWS", str(rows))
+    dm = DeviceModel.synthetic(cfg, seed=80 + H)
+    prompts = D.rng(81 + n).integers(0, cfg.V, size=(B, n)).astype(np.int32)
+    got = {}
+    for kind in ("tiled", "rows"):
+        monkeypatch.setenv("EF_HIP_PREFILL_ATTENTION", kind)
+        eng = Engine(dm, max_seq=n + 1, batch=B)
+        eng.prefill(prompts, 0)
+        got[kind] = eng.logits().copy()
+        eng.close()
+    assert _err(got["tiled"], got["rows"]) < 1e-5
