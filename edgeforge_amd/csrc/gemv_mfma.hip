@@ -1,4 +1,4 @@
-// Packed Q4_0 / Q8_0 GEMV on the matrix cores for batches of sequences (2..64 per launch).
+// Packed Q4_0 / Q8_0 GEMV on the matrix cores for batches of sequences.
 //
 // Two kernels per launch (three with a K split):
 //  1. xfrag_kernel turns the activations [B][K] (optionally RMS-normalised, kern::rmsnorm order)
@@ -908,6 +908,298 @@ __global__ __launch_bounds__(256) void finalize_kernel(FinArgs a) {
   if (a.em.on()) emit_block(a.em, sq, row >> 5, row & 31, out, live);
 }
 
+
+// ---- many sequences (a prefill's rows, teacher-forced scoring) --------------------------------------
+// The kernel above reads every A fragment from L2 once per 16 RT rows, which bounds it at a few hundred
+// sequences.  Here a workgroup of four waves owns NS sequence tiles and 64 rows (32 of each matrix for
+// SwiGLU) per 4 / KW waves; a stage is KW K blocks, one per group of 4 / KW waves.  Stages go from
+// memory to a ring of four LDS slots by LDS-DMA, three ahead of their use, and a stage's W and first A
+// fragments are read into registers while the stage before it is on the matrix cores.  The K shares
+// are combined through LDS in a fixed order.  Products and scales as block_products; every
+// kRowsFlush blocks the running sums move into a second set, so no chain of FP32 additions is long
+// (one chain over K = 2048 measured 2.5e-7 relative error against 2.1e-7 for the kernel above).
+constexpr int kRowUnits = 4;  // 16-row tiles (times matrices) per wave
+constexpr int kRowWaves = 4, kRT = kRowWaves * kWave;
+constexpr int kRowSlots = 4, kRowsFlush = 8;
+
+// One stage in LDS: KW NS sequence tiles' fragments, then 8 kRowUnits tile-blocks of W in whole KB; after
+// the slots, 1 KB that the DMA's surplus pieces are written to.
+__host__ __device__ constexpr uint32_t rows_stage_bytes(int ns, int kw, bool q4) {
+  return kw * ns * 2048u + (1u * kRowWaves * kRowUnits * (q4 ? kTileBlockQ4 : kTileBlockQ8) + 1023u) / 1024u * 1024u;
+}
+
+// 16 bytes per lane from src to LDS at dst + 16 lane, asynchronously (vmcnt).  Written as asm because the
+// compiler, seeing such a copy, waits for it before every later LDS read; the kernel waits for its
+// stages itself.  No register is written but m0, which the compiler sets anew before each use.
+__device__ __forceinline__ void dma16(uint32_t dst, const uint8_t* src) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory");
+}
+
+// At most N of this wave's DMA pieces still in flight and its LDS reads done, then the barrier.
+template <int N>
+__device__ __forceinline__ void stage_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int NM, int NS, int KW, bool Q4>
+__device__ __forceinline__ void rows_loop(const MJob& jb, const uint8_t* tab, int nb, int tile_row0, int tile0,
+                                          int wave, int lane, uint8_t* lb, f4v (&acc)[kRowUnits / NM][NM][NS]) {
+  constexpr int RT = kRowUnits / NM, RW = kRowWaves / KW, UW = RW * kRowUnits;
+  constexpr uint32_t bb = Q4 ? kTileBlockQ4 : kTileBlockQ8;
+  constexpr int P = static_cast<int>(bb / 16);
+  constexpr int kA = KW * NS * 128, kW = KW * UW * P;  // 16-byte pieces of a stage
+  constexpr int NA = (kA + kRT - 1) / kRT, NW = (kW + kRT - 1) / kRT, N = NA + NW;
+  constexpr uint32_t a_bytes = kA * 16, stage = rows_stage_bytes(NS, KW, Q4);
+  static_assert(stage == a_bytes + (kW + 63) / 64 * 1024, "stage layout");
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)lb));
+  const int last_tile = static_cast<int>(jb.bytes / (static_cast<uint32_t>(nb) * bb)) - 1;
+  // this thread's pieces: address in stage 0 and LDS offset (of the wave's lane 0) in a slot; rounds
+  // past the stage's pieces repeat its last ones into the spare KB
+  const uint8_t* src[N];
+  uint32_t dst[N];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+    const int w0 = wave * kWave + kRT * i;
+    const int q = (w0 < kA ? w0 : 0) + lane, kw = q / (NS * 128), r = q % (NS * 128);
+    src[i] = tab + (static_cast<size_t>(tile0 + r / 128) * nb + kw) * 2048u + (r % 128) * 16u;
+    dst[i] = w0 < kA ? w0 * 16u : kRowSlots * stage;
+  }
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    const int w0 = wave * kWave + kRT * i;
+    const int q = min((w0 < kW ? w0 : 0) + lane, kW - 1), kw = q / (UW * P), r = q % (UW * P), u = r / P;
+    const int tr = min(tile_row0 + u / NM, last_tile);
+    src[NA + i] = (NM == 2 && (u & 1) ? jb.W2 : jb.W) + (static_cast<size_t>(tr) * nb + kw) * bb + (r % P) * 16u;
+    dst[NA + i] = w0 < kW ? a_bytes + w0 * 16u : kRowSlots * stage;
+  }
+  const int nst = nb / KW;  // KW divides nb
+  int fetched = 0, fslot = 0;
+  auto fetch = [&]() {  // the next stage into the next slot; past the last stage, that one again
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      dma16(__builtin_amdgcn_readfirstlane(lds0 + dst[i] + (dst[i] == kRowSlots * stage ? 0u : fslot * stage)), src[i]);
+      const uint32_t inc = i < NA ? KW * 2048u : KW * bb;
+      src[i] += fetched + 1 < nst ? inc : 0u;
+    }
+    ++fetched;
+    fslot = (fslot + 1) % kRowSlots;
+  };
+  const int kw = wave / RW, rwv = wave % RW;
+  WRegs<Q4> W[kRowUnits];
+  auto read_w = [&](int slot) {
+    const uint8_t* pw = lb + static_cast<uint32_t>(slot) * stage + a_bytes +
+                        static_cast<uint32_t>(kw * UW + rwv * kRowUnits) * bb;
+#pragma unroll
+    for (int u = 0; u < kRowUnits; ++u) {
+      const uint8_t* p = pw + u * bb;
+      if constexpr (Q4) {
+        W[u].c0 = *reinterpret_cast<const uint32_t*>(p + lane * 4);
+        W[u].c1 = 0;
+      } else {
+        const uint2 v = *reinterpret_cast<const uint2*>(p + lane * 8);
+        W[u].c0 = v.x;
+        W[u].c1 = v.y;
+      }
+      W[u].sc = *reinterpret_cast<const uint16_t*>(p + (Q4 ? 256 : 512) + 2 * (lane & 15));
+    }
+  };
+  auto read_a = [&](h8 (&x)[2], int slot, int tile) {
+    const uint8_t* pa = lb + static_cast<uint32_t>(slot) * stage + kw * NS * 2048 + tile * 2048 + lane * 16;
+    x[0] = *reinterpret_cast<const h8*>(pa);
+    x[1] = *reinterpret_cast<const h8*>(pa + 1024);
+  };
+  auto operand = [&](int u) -> h8 { return Q4 ? q4_operand(W[u].c0) : q8_operand(W[u].c0, W[u].c1); };
+  fetch();
+  fetch();
+  fetch();
+  stage_barrier<2 * N>();
+  // The sequence tiles of all stages form one pipeline: while a tile's products with the wave's four row
+  // units run, the vector ALU adds the tile before it (of the stage before for the first) and converts
+  // the next stage's codes, and the next tile's fragments are read, so the matrix cores do not drain
+  // at a stage's end.
+  const f4v Z = {0.0f, 0.0f, 0.0f, 0.0f};
+  h8 B[2][kRowUnits], A[2][2];
+  uint32_t sc[2][kRowUnits];
+  read_w(0);
+  read_a(A[0], 0, 0);
+#pragma unroll
+  for (int u = 0; u < kRowUnits; ++u) {
+    B[0][u] = operand(u);
+    sc[0][u] = W[u].sc;
+    sc[1][u] = 0;
+  }
+  f4v Dp[kRowUnits] = {Z, Z, Z, Z};
+  f4v run[RT][NM][NS];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int mt = 0; mt < NM; ++mt)
+#pragma unroll
+      for (int t = 0; t < NS; ++t) run[rt][mt][t] = Z;
+  int slot = 0;
+  // ap: which A registers hold tile 0 (alternating when NS is odd); p: the parity of B and sc
+  auto step = [&](auto par) {
+    constexpr int p = decltype(par)::value, ap = NS % 2 ? p : 0;
+    stage_barrier<N>();  // the next stage has landed; every wave is done with the stage before
+    const int next = (slot + 1) % kRowSlots;
+    read_w(next);
+#pragma unroll
+    for (int t = 0; t < NS; ++t) {
+      constexpr int kPer = (kRowUnits + NS - 1) / NS;  // units of the next stage converted per tile
+      const int ca = (ap + t) & 1;
+      if (t + 1 < NS) {
+        read_a(A[1 - ca], slot, t + 1);
+      } else {
+        read_a(A[1 - ca], next, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      f4v D[kRowUnits];
+#pragma unroll
+      for (int u = 0; u < kRowUnits; ++u) D[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[ca][0], B[p][u], Z, 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < kRowUnits; ++u) D[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[ca][1], B[p][u], D[u], 0, 0, 0);
+      const int pt = t > 0 ? t - 1 : NS - 1;
+#pragma unroll
+      for (int u = 0; u < kRowUnits; ++u) {
+        const float d = f16lo(sc[t > 0 ? p : 1 - p][u]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) run[u / NM][u % NM][pt][r] = fmaf(d, Dp[u][r], run[u / NM][u % NM][pt][r]);
+      }
+#pragma unroll
+      for (int u = t * kPer; u < t * kPer + kPer; ++u)
+        if (u < kRowUnits) B[1 - p][u] = operand(u);
+      if (t == 0) {
+#pragma unroll
+        for (int u = 0; u < kRowUnits; ++u) sc[1 - p][u] = W[u].sc;
+      }
+#pragma unroll
+      for (int u = 0; u < kRowUnits; ++u) Dp[u] = D[u];
+#pragma unroll
+      for (int i = 0; i < 2 * kRowUnits; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                       // one product
+        __builtin_amdgcn_sched_group_barrier(0x002, (16 + 10 * kPer + 7) / 8, 0);  // vector ALU work
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (t == 0) {
+        fetch();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    slot = next;
+  };
+  auto flush = [&]() {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int mt = 0; mt < NM; ++mt)
+#pragma unroll
+        for (int t = 0; t < NS; ++t) {
+          acc[rt][mt][t] += run[rt][mt][t];
+          run[rt][mt][t] = Z;
+        }
+  };
+  for (int s0 = 0; s0 < nst; s0 += kRowsFlush) {
+    const int s1 = min(nst, s0 + kRowsFlush);
+    for (int st = s0; st < s1; st += 2) {
+      step(std::integral_constant<int, 0>{});
+      if (st + 1 < s1) step(std::integral_constant<int, 1>{});
+    }
+    if (s1 < nst) flush();
+  }
+  // the last tile of the last stage
+  const int lp = (nst - 1) & 1;
+#pragma unroll
+  for (int u = 0; u < kRowUnits; ++u) {
+    const float d = f16lo(lp ? sc[1][u] : sc[0][u]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) run[u / NM][u % NM][NS - 1][r] = fmaf(d, Dp[u][r], run[u / NM][u % NM][NS - 1][r]);
+  }
+  flush();
+  // no DMA may land in the LDS the epilogue (or the next workgroup of the CU) uses
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+template <int NM, int NS, int KW>
+__global__ __launch_bounds__(kRT, 2) void gemv_rows_kernel(MArgs a, int groups, int sgs, int residual) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lb[];
+  constexpr int RT = kRowUnits / NM, RW = kRowWaves / KW, ROWS = RW * RT * kTileRows;
+  // Workgroup ids go round the 8 XCDs: each XCD takes a contiguous run of the order (8 sequence groups)
+  // x (row groups) x (the 8), so the workgroups it holds at a time share their A and W through its L2.
+  const int total = groups * sgs, per = (total + 7) / 8;
+  const int lin = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
+  if (lin >= total) return;
+  const int sc = lin / (8 * groups), in = lin - sc * 8 * groups, wide = min(8, sgs - sc * 8);
+  const int grp = in / wide, sg = sc * 8 + in % wide;
+  const MJob jb = find_mjob(a, grp);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+  const int row0 = (grp - jb.tile_begin) * ROWS, nb = a.K >> 5;
+  const bool q4 = jb.qtype == EF_QTYPE_Q4_0;
+  f4v acc[RT][NM][NS];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int mt = 0; mt < NM; ++mt)
+#pragma unroll
+      for (int t = 0; t < NS; ++t) acc[rt][mt][t] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+  if (q4) {
+    rows_loop<NM, NS, KW, true>(jb, a.t4, nb, row0 / kTileRows, sg * NS, wave, lane, lb, acc);
+  } else {
+    rows_loop<NM, NS, KW, false>(jb, a.t8, nb, row0 / kTileRows, sg * NS, wave, lane, lb, acc);
+  }
+  const int j = lane & 15, g = lane >> 4, rwv = wave % RW, kw = wave / RW;
+  auto finish = [&](int rt, int t, const f4v (&v)[NM]) {
+    const int row = row0 + (rwv * RT + rt) * kTileRows + j;
+    if (row >= jb.rows) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int sq = (sg * NS + t) * kSeqTile + 4 * g + r;
+      if (sq >= a.B) break;
+      const float post = a.post[sq];
+      float* y = jb.y + sq * jb.ldy + row;
+      if (NM == 2) {
+        *y = silu_m(v[0][r] * post) * (v[NM - 1][r] * post);
+      } else {
+        *y = residual ? *y + v[0][r] * post : v[0][r] * post;
+      }
+    }
+  };
+  if constexpr (KW == 1) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int t = 0; t < NS; ++t) {
+        f4v v[NM];
+#pragma unroll
+        for (int mt = 0; mt < NM; ++mt) v[mt] = acc[rt][mt][t];
+        finish(rt, t, v);
+      }
+  } else {
+    constexpr int F = RT * NS;  // fragments (per matrix) of a wave
+    f4v* red = reinterpret_cast<f4v*>(lb);  // [row wave][K share][fragment][matrix][lane]
+    __syncthreads();
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int t = 0; t < NS; ++t)
+#pragma unroll
+        for (int mt = 0; mt < NM; ++mt)
+          red[((rwv * KW + kw) * F + rt * NS + t) * NM * kWave + mt * kWave + lane] = acc[rt][mt][t];
+    __syncthreads();
+    for (int f = kw; f < F; f += KW) {
+      f4v v[NM];
+#pragma unroll
+      for (int mt = 0; mt < NM; ++mt) {
+        v[mt] = red[(rwv * KW * F + f) * NM * kWave + mt * kWave + lane];
+#pragma unroll
+        for (int k = 1; k < KW; ++k) v[mt] += red[((rwv * KW + k) * F + f) * NM * kWave + mt * kWave + lane];
+      }
+      finish(f / NS, f % NS, v);
+    }
+  }
+}
+
 // (RT, NS) shapes the kernels are instantiated for: the ones whose registers fit in 256 VGPRs
 // (two waves per SIMD) without spilling.  SwiGLU keeps two accumulators per output.
 struct Shape {
@@ -947,6 +1239,7 @@ struct Plan {
   int nm = 1, NT = 1, RT = 2, NS = 1, SG = 1, groups = 0, S = 1, bps = 0, chunk = 0;
   size_t tab = 0, part_off = 0, bytes = 0, lds = 0;
   double cost = 0.0;
+  bool rows = false;  // the many-sequence kernel (plan_rows per launch)
 };
 
 int groups_for(const GemvJob* jobs, int n_jobs, int rows_wg) {
@@ -979,8 +1272,68 @@ double shape_cost(int rt, int nm, int ns, int sg, int groups, int S, int bps, si
   return t;
 }
 
-// even_rt: only shapes whose workgroup rows are a multiple of 32 (outputs staged as tables).
-Plan plan_mfma(const GemvJob* jobs, int n_jobs, int epi, int batch, size_t ldx, bool even_rt = false) {
+
+// The many-sequence kernel's launches: at most kRowsMax sequences, from kRowsFrom sequences and
+// kRowsMacs multiply-adds on (weight rows x matrices x sequences x K).  Below that its workgroups leave
+// CUs idle and the split-K kernel is the faster one; us per call, split-K / this one: 2048x2048 Q4_0
+// 500 sequences (2.1G) 28 / 33, 2048x5632 200 (2.3G) 37 / 39; SwiGLU 5632x2048 200 (4.6G) 52 / 47, 500
+// 80 / 73, 1500 214 / 184, 2048x5632 500 (5.8G) 62 / 57, 1024 109 / 90, 2048x2048 1500 (6.3G) 71 / 56,
+// Q8_0 32000x2048 200 (13G) 122 / 87, 510 228 / 164.
+constexpr int kRowsMax = 4096, kRowsFrom = 128;
+constexpr double kRowsMacs = 3.5e9;
+int rows_tiles(int rows) { return ((rows + kSeqTile - 1) / kSeqTile + 11) / 12 * 12; }  // a multiple of every NS
+
+// The kernel's instantiated shapes (sequence tiles, K shares per workgroup) and their measured times
+// per stage in us, one workgroup on a CU and two (two need half the LDS each).
+struct RowsShape {
+  int NS, KW;
+  float t1, t2;
+};
+constexpr RowsShape kRowsShapes[] = {{4, 1, 0.66f, 1.03f}, {3, 1, 0.59f, 0.88f}, {4, 2, 0.77f, 1.30f},
+                                     {3, 2, 0.68f, 0.98f}, {2, 2, 0.59f, 0.90f}, {4, 4, 1.05f, 2.00f},
+                                     {2, 4, 0.71f, 1.25f}};
+
+struct RowsPlan {
+  int NS = 0, KW = 1, groups = 0, sgs = 0;
+  size_t lds = 0;
+};
+
+template <int NM>
+void* pick_rows(int ns, int kw) {
+  auto kf = [](auto* f) { return reinterpret_cast<void*>(f); };
+  if (kw == 1) return ns == 4 ? kf(&gemv_rows_kernel<NM, 4, 1>) : kf(&gemv_rows_kernel<NM, 3, 1>);
+  if (kw == 4) return ns == 4 ? kf(&gemv_rows_kernel<NM, 4, 4>) : kf(&gemv_rows_kernel<NM, 2, 4>);
+  return ns == 4 ? kf(&gemv_rows_kernel<NM, 4, 2>)
+                 : (ns == 3 ? kf(&gemv_rows_kernel<NM, 3, 2>) : kf(&gemv_rows_kernel<NM, 2, 2>));
+}
+
+// The shape of the least estimated time for `rows` sequences: workgroups are dealt to the CUs evenly,
+// two to a CU at a time when their LDS allows it, plus 8 us per pair for its ends.
+RowsPlan plan_rows(const GemvJob* jobs, int n_jobs, int nm, int rows, bool q8) {
+  RowsPlan best;
+  const int cus = ctx().cu_count > 0 ? ctx().cu_count : 256, nb = static_cast<int>(jobs[0].W->cols / 32);
+  const size_t lim = ctx().lds_per_block > 0 ? ctx().lds_per_block : 65536;
+  const int NT = (rows + kSeqTile - 1) / kSeqTile;
+  double cost = 0.0;
+  for (const RowsShape& sh : kRowsShapes) {
+    const size_t lds = std::max(size_t(kRowSlots) * rows_stage_bytes(sh.NS, sh.KW, !q8) + 1024,
+                                sh.KW > 1 ? static_cast<size_t>(kRowWaves) * kRowUnits * sh.NS * kWave * 16 : 0);
+    if (nb % sh.KW != 0 || lds > lim) continue;
+    const int groups = groups_for(jobs, n_jobs, kRowWaves / sh.KW * kRowUnits / nm * kTileRows);
+    const int sgs = (NT + sh.NS - 1) / sh.NS;
+    const int per_cu = (groups * sgs + cus - 1) / cus, pairs = per_cu / 2, odd = per_cu % 2;
+    const double c = nb / sh.KW * (pairs * (2 * lds <= lim ? sh.t2 : 2 * sh.t1) + odd * sh.t1) + 8.0 * (pairs + odd);
+    if (best.NS != 0 && c >= cost) continue;
+    cost = c;
+    best = RowsPlan{sh.NS, sh.KW, groups, sgs, lds};
+  }
+  return best;
+}
+
+// staged: the launch reads producer-staged tables (never the many-sequence kernel); even_rt: only shapes
+// whose workgroup rows are a multiple of 32 (outputs staged as tables).
+Plan plan_mfma(const GemvJob* jobs, int n_jobs, int epi, int batch, size_t ldx, bool staged = false,
+               bool even_rt = false) {
   Plan p;
   if (batch < 2 || n_jobs < 1 || n_jobs > kMaxJobsM) return p;
   const size_t K = jobs[0].W->cols;
@@ -997,6 +1350,22 @@ Plan plan_mfma(const GemvJob* jobs, int n_jobs, int epi, int batch, size_t ldx, 
   const size_t xld = jobs[0].ldx ? jobs[0].ldx : ldx;
   if (reinterpret_cast<uintptr_t>(jobs[0].x) % 16 != 0 || xld % 4 != 0) return p;
   p.nm = epi == kEpiSwiglu ? 2 : 1;
+  // decided by the count of 16-sequence tiles, so workspaces sized by tile counts hold for every batch
+  const int padded = (batch + kSeqTile - 1) / kSeqTile * kSeqTile;
+  double macs = 0.0;
+  for (int j = 0; j < n_jobs; ++j) macs += static_cast<double>(jobs[j].W->rows) * p.nm * padded * K;
+  if (!staged && padded >= kRowsFrom && macs >= kRowsMacs) {
+    // A tables of every sequence tile a shape may round up to (zeros past the batch)
+    const int chunk = std::min(batch, kRowsMax), tiles = rows_tiles(chunk);
+    const size_t tab = static_cast<size_t>(tiles) * (K / 32) * 2 * kWave * 16;
+    if (tab < (size_t(1) << 32) && static_cast<size_t>(chunk) * xld * 4 < (size_t(1) << 32)) {
+      p.rows = p.ok = true;
+      p.chunk = chunk;
+      p.tab = tab;
+      p.bytes = (p.q4 ? tab : 0) + (p.q8 ? tab : 0) + static_cast<size_t>(tiles) * kSeqTile * sizeof(float);
+      return p;
+    }
+  }
   p.chunk = std::min(batch, kMaxTiles * kSeqTile);
   p.NT = (p.chunk + kSeqTile - 1) / kSeqTile;
   const int nb = static_cast<int>(K / 32);
@@ -1100,8 +1469,6 @@ int ensure_tiled(const ef_hip_weight_s* w, hipStream_t s) {
   return EF_HIP_OK;
 }
 
-int gemv_mfma_max_rows() { return kMaxTiles * kSeqTile; }
-
 size_t gemv_mfma_workspace_bytes(const GemvJob* jobs, int n_jobs, int epi, int batch, size_t ldx) {
   const Plan p = plan_mfma(jobs, n_jobs, epi, batch, ldx);
   return p.ok ? p.bytes : 0;
@@ -1136,10 +1503,10 @@ int launch_gemv_mfma(const GemvJob* jobs, int n_jobs, int epi, const float* norm
   a.ksplit = pl.S;
   a.blocks_per_split = pl.bps;
   a.part = reinterpret_cast<float*>(base + pl.part_off);
-  void* fn = epi == kEpiStore ? pick_mfma<kEpiStore>(pl.RT, pl.NS)
-                              : (epi == kEpiResidual ? pick_mfma<kEpiResidual>(pl.RT, pl.NS)
-                                                     : pick_mfma<kEpiSwiglu>(pl.RT, pl.NS));
-  const int rows_wg = pl.RT * kTileRows;
+  void* fn = pl.rows ? nullptr
+             : epi == kEpiStore ? pick_mfma<kEpiStore>(pl.RT, pl.NS)
+                                : (epi == kEpiResidual ? pick_mfma<kEpiResidual>(pl.RT, pl.NS)
+                                                       : pick_mfma<kEpiSwiglu>(pl.RT, pl.NS));
   for (int b0 = 0; b0 < batch && rc == EF_HIP_OK; b0 += pl.chunk) {
     const int nb = std::min(pl.chunk, batch - b0);
     PrepArgs p{};
@@ -1153,11 +1520,14 @@ int launch_gemv_mfma(const GemvJob* jobs, int n_jobs, int epi, const float* norm
     p.t8 = t8;
     p.post = post;
     const int nbk = static_cast<int>(K / 32);
-    if (K <= static_cast<size_t>(kSeqPrepMaxK)) {  // tiles past B get zeros
-      hipLaunchKernelGGL(xfrag_seq_kernel, dim3(pl.SG * pl.NS * kSeqTile), dim3(kSeqPrepThreads), 0, stream, p);
+    const RowsPlan rp = pl.rows ? plan_rows(jobs, n_jobs, pl.nm, nb, pl.q8) : RowsPlan{};
+    const int rows_wg = pl.rows ? kRowWaves / rp.KW * kRowUnits / pl.nm * kTileRows : pl.RT * kTileRows;
+    const int prep_tiles = pl.rows ? rp.sgs * rp.NS : pl.SG * pl.NS;  // tiles past B get zeros
+    if (K <= static_cast<size_t>(kSeqPrepMaxK)) {
+      hipLaunchKernelGGL(xfrag_seq_kernel, dim3(prep_tiles * kSeqTile), dim3(kSeqPrepThreads), 0, stream, p);
     } else {
-      hipLaunchKernelGGL(xfrag_kernel, dim3((nbk + kPrepBlocks - 1) / kPrepBlocks, pl.SG * pl.NS), dim3(kTP), 0,
-                         stream, p);
+      hipLaunchKernelGGL(xfrag_kernel, dim3((nbk + kPrepBlocks - 1) / kPrepBlocks, prep_tiles), dim3(kTP), 0, stream,
+                         p);
     }
     a.n_jobs = n_jobs;
     a.K = static_cast<int>(K);
@@ -1180,6 +1550,14 @@ int launch_gemv_mfma(const GemvJob* jobs, int n_jobs, int epi, const float* norm
       d.ldy = static_cast<long>(yld);
       d.tile_begin = tiles;
       tiles += (d.rows + rows_wg - 1) / rows_wg;
+    }
+    if (pl.rows) {
+      int groups = rp.groups, sgs = rp.sgs, residual = epi == kEpiResidual ? 1 : 0;
+      void* rparams[] = {&a, &groups, &sgs, &residual};
+      const hipError_t e = hipLaunchKernel(pl.nm == 2 ? pick_rows<2>(rp.NS, rp.KW) : pick_rows<1>(rp.NS, rp.KW),
+                                           dim3((groups * sgs + 7) / 8 * 8), dim3(kRT), rparams, rp.lds, stream);
+      if (e != hipSuccess) rc = fail_hip(e, "gemv_rows_kernel");
+      continue;
     }
     void* params[] = {&a};
     // the chunk's sequences cover ceil(nb / 16) tiles; grid rows past them would have no sequences
@@ -1217,7 +1595,7 @@ int launch_gemv_mfma(const GemvJob* jobs, int n_jobs, int epi, const float* norm
 
 
 size_t gemv_mfma_staged_workspace_bytes(const GemvJob* jobs, int n_jobs, int epi, int batch, bool emit) {
-  const Plan p = plan_mfma(jobs, n_jobs, epi, batch, jobs[0].W->cols, emit);
+  const Plan p = plan_mfma(jobs, n_jobs, epi, batch, jobs[0].W->cols, true, emit);
   return p.ok ? p.bytes : 0;
 }
 
@@ -1253,7 +1631,7 @@ int launch_gemv_mfma_staged(const GemvJob* jobs, int n_jobs, int epi, const Mfma
                             void* ws, size_t ws_bytes, hipStream_t stream, const AEmit* em) {
   const size_t K = jobs[0].W->cols;
   const bool emit = em != nullptr && em->on();
-  const Plan pl = plan_mfma(jobs, n_jobs, epi, batch, K, emit);
+  const Plan pl = plan_mfma(jobs, n_jobs, epi, batch, K, true, emit);
   if (emit) {
     EFH_CHECK(n_jobs == 1 && jobs[0].W->rows % 32 == 0 && static_cast<int>(jobs[0].W->rows / 32) == em->nb &&
                   em->bpad >= stage_bpad(batch),

@@ -182,3 +182,65 @@ def test_refresh_after_rewriting_device_bytes(hip, qtype):
     y1 = hip.DeviceArray((rows,))
     hip.matvec(W, hip.DeviceArray.from_host(X[0]), y1, batch=1)
     assert np.abs(y1.numpy() - got[0]).max() <= ABS_TOL + 1e-5 * np.abs(got[0]).max()
+
+
+def _exact_close(W64, X, got, what):
+    """|got - exact| <= 1e-5 * sum|w x| for every output (the single-vector gate)."""
+    x = X.astype(np.float64)
+    err = np.abs(got - x @ W64.T) / np.maximum(np.abs(x) @ np.abs(W64).T, 1e-30)
+    assert err.max() < REL_TOL, (what, float(err.max()))
+
+
+@pytest.mark.parametrize("qtype,rows,cols,batch", [
+    (O.Q4_0, 2001, 2080, 900),   # an odd count of K blocks (65), a partial row tile, 57 sequence tiles
+    (O.Q8_0, 2001, 2048, 900),
+    (O.Q4_0, 600, 5632, 1100),   # long rows, few row groups: K shares
+    (O.Q4_0, 3401, 256, 4100),   # two launches, the second of 4 sequences; 8 K blocks (one flush)
+    (O.Q8_0, 15000, 2048, 129),  # one sequence past a tile
+])
+def test_many_sequence_kernel_edges(hip, qtype, rows, cols, batch):
+    """The many-sequence kernel (3.5G multiply-adds or more in a call) at the edges of its tiles."""
+    print(f"[case] many-sequence gemv qtype={qtype} {rows}x{cols} B={batch}", flush=True)
+    packed = D.random_rows(qtype, rows, cols, seed=rows + batch)
+    X = (D.rng(rows).standard_normal((batch, cols)) * np.exp(D.rng(cols).normal(size=(batch, 1)))).astype(np.float32)
+    W = hip.Weight(qtype, rows, cols, host=packed)
+    dx, dy = hip.DeviceArray.from_host(X), hip.DeviceArray((batch, rows))
+    hip.matvec(W, dx, dy, batch=batch)
+    got = dy.numpy()
+    w64 = D.dequant_exact(qtype, packed, cols)
+    _exact_close(w64, X, got, "store")
+    base = D.rng(3).standard_normal((batch, rows)).astype(np.float32)
+    dy.upload(base)
+    hip.matvec_residual(W, dx, dy, batch=batch)
+    # the same sums added to y: one more rounding of the result
+    assert np.abs(dy.numpy() - (base + got)).max() <= 2.0 ** -23 * (np.abs(base) + np.abs(got)).max()
+
+
+def test_many_sequence_kernel_swiglu_and_mixed_jobs(hip):
+    K, F, B = 2048, 1000, 900
+    rng = D.rng(77)
+    X = rng.standard_normal((B, K)).astype(np.float32)
+    nw = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    x64 = X.astype(np.float64)
+    h = nw * (x64 / np.sqrt((x64 * x64).mean(1, keepdims=True) + 1e-5))
+    dx, dn = hip.DeviceArray.from_host(X), hip.DeviceArray.from_host(nw)
+    pk = [D.random_rows(O.Q4_0, F, K, seed=90 + i) for i in range(2)]
+    G, U = [hip.Weight(O.Q4_0, F, K, host=p) for p in pk]
+    dy = hip.DeviceArray((B, F))
+    hip.matvec_swiglu(G, U, dx, dy, dn, 1e-5, batch=B)
+    g, u = [h @ D.dequant_exact(O.Q4_0, p, K).T for p in pk]
+    sg, su = [np.abs(h) @ np.abs(D.dequant_exact(O.Q4_0, p, K)).T for p in pk]
+    want = g / (1 + np.exp(-g)) * u
+    # each factor within 1e-5 of its sum of |w x| (|silu'| < 1.1), plus the FP32 rounding of the product
+    bound = 1e-5 * (1.1 * sg * np.abs(u) + np.abs(g) * su) + 1e-6 * np.abs(want) + 1e-10 * sg * su
+    assert (np.abs(dy.numpy() - want) <= bound).all()
+    jobs, mats = [], []
+    for i, (qt, rows) in enumerate([(O.Q4_0, 2048), (O.Q8_0, 130), (O.Q4_0, 70)]):
+        p = D.random_rows(qt, rows, K, seed=95 + i)
+        y = hip.DeviceArray((B, 2048))
+        jobs.append((hip.Weight(qt, rows, K, host=p), dx, y))
+        mats.append(D.dequant_exact(qt, p, K))
+    hip.matvec_jobs_rmsnorm(jobs, dn, 1e-5, batch=B, ldx=K, ldy=2048)
+    for (W, _, y), w64 in zip(jobs, mats):
+        err = np.abs(y.numpy()[:, :W.rows] - h @ w64.T) / np.maximum(np.abs(h) @ np.abs(w64).T, 1e-30)
+        assert err.max() < REL_TOL
