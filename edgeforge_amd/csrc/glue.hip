@@ -1002,6 +1002,169 @@ __global__ __launch_bounds__(kSplitThreads) void attention_combine_kernel(AttnAr
   }
 }
 
+// Decode attention of a large batch (hd = 64, at most 16 query heads per KV head): one workgroup per
+// (KV group, sequence), as attention_group_kernel, but one pass with a running
+// maximum and no staging: the eight waves take 32-position chunks in turn and read their K and V rows
+// straight into operands of v_mfma_f32_16x16x4_f32 (prefill_mfma_kernel's layouts and sums, the pairs
+// being the group's heads; columns past them idle).  A chunk's K registers are refilled once its
+// scores are formed and its V registers once they are used, so each wave keeps a chunk in flight.
+// The waves' sums are combined through LDS in wave order.
+//
+// Bound by reading the cache, 2 x 256 bytes per position and workgroup: 30.0 us per layer at position 900
+// of 64 sequences x 4 groups (118 MB, 3.9 TB/s; a large copy reaches 5.1), where the KV-group kernel,
+// which stages each 64-position chunk between barriers in two passes, took 77.7; 50.9 / 153.8 at 1900,
+// 8.3 / 12.2 at 100, 7.4 / 7.8 at 63.
+constexpr int kBatchThreads = 512, kBatchWaves = kBatchThreads / kWave, kBatchChunk = 32, kBatchHeads = 16, kBatchLd = 68;
+
+__global__ __launch_bounds__(kBatchThreads) void attention_batch_kernel(AttnArgs a) {
+  __shared__ float so[kBatchWaves][kBatchHeads * kBatchLd];
+  __shared__ float sm[kBatchWaves][kBatchHeads];
+  __shared__ double sl[kBatchWaves][kBatchHeads];
+  const int kv = blockIdx.x, b = blockIdx.y, t = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t / kWave), lane = t & (kWave - 1), m = lane & 15, g = lane >> 4;
+  const int hpg = a.H / a.KV, kvd = a.KV * 64;
+  const long seq0 = static_cast<long>(b) * a.max_seq * kvd + kv * 64;
+  const float* kc = a.kcache + seq0;
+  const float* vc = a.vcache + seq0;
+  f4n k[2][4], v[2][4];  // K: position 16 pt + m, dims 16 j + 4 g ..; V: position 16 pt + 4 g + r, dims 4 m ..
+  auto fetch_k = [&](int c0, int lim) {
+#pragma unroll
+    for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        k[pt][j] = *reinterpret_cast<const f4n*>(kc + static_cast<long>(min(c0 + 16 * pt + m, lim)) * kvd + 16 * j + 4 * g);
+  };
+  auto fetch_v = [&](int c0, int lim) {
+#pragma unroll
+    for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        v[pt][r] = *reinterpret_cast<const f4n*>(vc + static_cast<long>(min(c0 + 16 * pt + 4 * g + r, lim)) * kvd + 4 * m);
+  };
+  // the first chunk is requested before the position is known (every row of the cache is in bounds)
+  fetch_k(wave * kBatchChunk, a.max_seq - 1);
+  fetch_v(wave * kBatchChunk, a.max_seq - 1);
+  // RoPE in the operands' layout: dims i = 16 j + 4 g + s and i + 32 are in the same lane
+  f4n q[4], kn[4];
+  const float* qp = a.q + static_cast<long>(b) * a.ldq + (kv * hpg + min(m, hpg - 1)) * 64 + 4 * g;
+  const float* kp = a.knew + static_cast<long>(b) * kvd + kv * 64 + 4 * g;
+  const f4n vn = *reinterpret_cast<const f4n*>(a.vnew + static_cast<long>(b) * kvd + kv * 64 + 4 * m);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const f4n c = *reinterpret_cast<const f4n*>(a.rope_now + 16 * j + 4 * g);
+    const f4n s = *reinterpret_cast<const f4n*>(a.rope_now + 32 + 16 * j + 4 * g);
+    const f4n qa = *reinterpret_cast<const f4n*>(qp + 16 * j), qb = *reinterpret_cast<const f4n*>(qp + 32 + 16 * j);
+    const f4n ka = *reinterpret_cast<const f4n*>(kp + 16 * j), kb = *reinterpret_cast<const f4n*>(kp + 32 + 16 * j);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      q[j][e] = qa[e] * c[e] - qb[e] * s[e];
+      q[j + 2][e] = qb[e] * c[e] + qa[e] * s[e];
+      kn[j][e] = ka[e] * c[e] - kb[e] * s[e];
+      kn[j + 2][e] = kb[e] * c[e] + ka[e] * s[e];
+    }
+  }
+  const int pos = *a.pos_dev;
+  if (wave == 0) {  // k / v at pos for later steps
+    float* kw = a.kcache + seq0 + static_cast<long>(pos) * kvd;
+    float* vw = a.vcache + seq0 + static_cast<long>(pos) * kvd;
+    if (m == 0) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<f4n*>(kw + 16 * j + 4 * g) = kn[j];
+    }
+    if (g == 0) *reinterpret_cast<f4n*>(vw + 4 * m) = vn;
+  }
+  const float c2 = a.scale * 1.44269504088896340736f;  // exponentials as 2^(c2 (s - max))
+  const f4n zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f4n o[4] = {zero, zero, zero, zero};
+  float mx = -INFINITY, sub = 0.0f;
+  double l = 0.0;
+  for (int c0 = wave * kBatchChunk; c0 <= pos; c0 += kBatchWaves * kBatchChunk) {
+    const int next = c0 + kBatchWaves * kBatchChunk;
+    f4n sc[2];
+#pragma unroll
+    for (int pt = 0; pt < 2; ++pt) {
+      const bool cur = c0 + 16 * pt + m == pos;
+      f4n part[2] = {zero, zero};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          part[j / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur ? kn[j][e] : k[pt][j][e], q[j][e], part[j / 2], 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sc[pt][r] = c0 + 16 * pt + 4 * g + r <= pos ? part[0][r] + part[1][r] : -INFINITY;
+    }
+    if (next <= pos) fetch_k(next, pos);
+    float cm = -INFINITY;
+#pragma unroll
+    for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) cm = fmaxf(cm, sc[pt][r]);
+    cm = fmaxf(cm, __shfl_xor(cm, 16, kWave));
+    cm = fmaxf(cm, __shfl_xor(cm, 32, kWave));
+    float al = 1.0f;
+    if (__any(cm > mx)) {
+      const float nm = fmaxf(mx, cm);
+      sub = nm == -INFINITY ? 0.0f : nm * c2;
+      al = __builtin_amdgcn_exp2f(fmaf(mx, c2, -sub));
+      l *= static_cast<double>(al);
+      mx = nm;
+    }
+    f4n oc[4] = {zero, zero, zero, zero};  // the chunk's own p.v
+#pragma unroll
+    for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int p = c0 + 16 * pt + 4 * g + r;
+        const float e = __builtin_amdgcn_exp2f(fmaf(sc[pt][r], c2, -sub));
+        l += static_cast<double>(e);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const float vv = p == pos ? vn[d] : (p < pos ? v[pt][r][d] : 0.0f);
+          oc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv, e, oc[d], 0, 0, 0);
+        }
+      }
+    if (next <= pos) fetch_v(next, pos);
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[d][r] = fmaf(o[d][r], al, oc[d][r]);
+  }
+  l += __shfl_xor(l, 16, kWave);
+  l += __shfl_xor(l, 32, kWave);
+  // lane (m, g): dims 16 g + 4 r + d of head m
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    *reinterpret_cast<f4n*>(so[wave] + m * kBatchLd + 16 * g + 4 * r) = f4n{o[0][r], o[1][r], o[2][r], o[3][r]};
+  if (g == 0) {
+    sm[wave][m] = mx;
+    sl[wave][m] = l;
+  }
+  __syncthreads();
+  float* out = a.ctx + static_cast<long>(b) * a.ldq + kv * hpg * 64;
+  for (int idx = t; idx < hpg * 64; idx += kBatchThreads) {  // whole waves: hpg * 64 is a multiple of 64
+    const int hh = idx >> 6, d = idx & 63;
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kBatchWaves; ++w) M = fmaxf(M, sm[w][hh]);
+    const float ms = M == -INFINITY ? 0.0f : M * c2;
+    float acc = 0.0f;
+    double L = 0.0;
+#pragma unroll
+    for (int w = 0; w < kBatchWaves; ++w) {
+      const float f = __builtin_amdgcn_exp2f(fmaf(sm[w][hh], c2, -ms));  // 0 for a wave without a position
+      acc = fmaf(so[w][hh * kBatchLd + d], f, acc);
+      L += sl[w][hh] * static_cast<double>(f);
+    }
+    const float r = acc * static_cast<float>(1.0 / L);
+    out[idx] = r;
+    if (a.em.on()) {
+      const int e = kv * hpg * 64 + idx;
+      emit_block(a.em, b, e >> 5, e & 31, r, true);
+    }
+  }
+}
+
 // Prefill, step 1: every row r = (sequence b, chunk index i) at position p = *pos_dev + i gets RoPE
 // on each query head in place and on each key head, and its roped key and its value row are
 // written into the cache at p (the decode kernel's rotation, operation for operation).
@@ -1378,6 +1541,14 @@ int launch_attention(const AttnArgs& a, int batch, hipStream_t s) {
   const size_t lim = std::max<size_t>(ctx().lds_per_block, 65536);
   const int cus = ctx().cu_count > 0 ? ctx().cu_count : 256;
   const int choice = attention_choice();
+  // the KV-group kernel's launches at hd = 64 (unless a kernel is forced): the matrix-core pass, faster at
+  // every position measured
+  if (choice == 0 && a.hd == 64 && a.rope_now != nullptr && a.ldq % 4 == 0 && a.H / a.KV <= kBatchHeads &&
+      attention_uses_group(a, batch)) {
+    hipLaunchKernelGGL(attention_batch_kernel, dim3(a.KV, batch), dim3(kBatchThreads), 0, s, a);
+    EFH_HIP(hipGetLastError());
+    return EF_HIP_OK;
+  }
   if (attention_uses_group(a, batch)) {
     const int hpg = a.H / a.KV;
     EFH_CHECK(!a.em.on() || (hpg * a.hd) % 32 == 0, "attention: staging needs H / KV * hd % 32 == 0");

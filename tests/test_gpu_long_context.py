@@ -107,3 +107,34 @@ def test_position_split_equals_single_pass_within_tolerance(hip, B, monkeypatch)
     assert out["split"][0][0].tolist() == want.tolist()
     for k in range(20):
         assert _logit_err(out["split"][1][k][0], want_logits[k]) < 1e-4, k
+
+
+@pytest.mark.parametrize("H,KV,B", [(4, 2, 64), (8, 1, 130)])
+def test_large_batch_attention(hip, monkeypatch, H, KV, B):
+    """A large batch's steps run one matrix-core pass over the cache: its logits against the KV-group
+    kernel's within 1e-5 relative (FP32 sums in another order, as the position split above), at the
+    first positions, at the ends of the 32-position chunks (a chunk of one position, a full one) and
+    of the eight waves' round of them (256)."""
+    cfg = Config(D=64 * H, F=512, H=H, KV=KV, hd=64, V=256, L=2, max_pos=512)
+    print(f"[case] large-batch attention H={H} KV={KV} B={B}", flush=True)
+    dm = DeviceModel.synthetic(cfg, seed=90 + H)
+    ids = D.rng(91).integers(0, cfg.V, size=(B, 300)).astype(np.int32)
+    got = {}
+    for kind in ("auto", "group"):
+        if kind == "group":
+            monkeypatch.setenv("EF_HIP_ATTENTION", "group")
+        else:
+            monkeypatch.delenv("EF_HIP_ATTENTION", raising=False)
+        eng = Engine(dm, max_seq=300, batch=B)
+        got[kind] = []
+        done = 0
+        for first, last in ((0, 2), (30, 34), (222, 225), (254, 258), (287, 290)):
+            if first > done:
+                eng.prefill(ids[:, done:first], done)
+            for p in range(first, last):
+                eng.forward(ids[:, p], p)
+                got[kind].append(eng.logits().copy())
+            done = last
+        eng.close()
+    for a, b in zip(got["auto"], got["group"]):
+        assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
