@@ -105,6 +105,8 @@ int ef_hip_init(int device) {
 int ef_hip_shutdown(void) {
   if (!g_ctx.ready) return EF_HIP_OK;
   EFH_HIP(hipStreamSynchronize(g_ctx.stream));
+  EFH_RC(release_gemv_workspace(g_ctx.stream));
+  EFH_HIP(hipStreamSynchronize(g_ctx.stream));
   EFH_HIP(hipStreamDestroy(g_ctx.stream));
   g_ctx = Context{};
   return EF_HIP_OK;

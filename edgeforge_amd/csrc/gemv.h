@@ -34,6 +34,8 @@ size_t gemv_mfma_workspace_bytes(const GemvJob* jobs, int n_jobs, int epi, int b
 size_t tiled_bytes(const ef_hip_weight_s* w);
 int ensure_tiled(const ef_hip_weight_s* w, hipStream_t s);
 int refresh_tiled(const ef_hip_weight_s* w, hipStream_t s);
+// Gives back the workspace kept for calls on the library's stream (which has drained).
+int release_gemv_workspace(hipStream_t stream);
 int launch_gemv_mfma(const GemvJob* jobs, int n_jobs, int epi, const float* norm_w, float eps, int batch, size_t ldx,
                      size_t ldy, void* ws, size_t ws_bytes, hipStream_t stream, bool* taken);
 

@@ -43,6 +43,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 
 #include "afrag.h"
 #include "gemv.h"
@@ -1330,26 +1331,38 @@ RowsPlan plan_rows(const GemvJob* jobs, int n_jobs, int nm, int rows, bool q8) {
   return best;
 }
 
-// staged: the launch reads producer-staged tables (never the many-sequence kernel); even_rt: only shapes
-// whose workgroup rows are a multiple of 32 (outputs staged as tables).
-Plan plan_mfma(const GemvJob* jobs, int n_jobs, int epi, int batch, size_t ldx, bool staged = false,
-               bool even_rt = false) {
-  Plan p;
-  if (batch < 2 || n_jobs < 1 || n_jobs > kMaxJobsM) return p;
-  const size_t K = jobs[0].W->cols;
-  if (K % 32 != 0 || K > 65536) return p;
-  size_t wbytes = 0;
-  for (int j = 0; j < n_jobs; ++j) {
-    if (jobs[j].W->qtype != EF_QTYPE_Q4_0 && jobs[j].W->qtype != EF_QTYPE_Q8_0) return Plan{};
-    p.q4 = p.q4 || jobs[j].W->qtype == EF_QTYPE_Q4_0;
-    p.q8 = p.q8 || jobs[j].W->qtype == EF_QTYPE_Q8_0;
-    wbytes += jobs[j].W->rows * jobs[j].W->row_bytes * (jobs[j].W2 ? 2 : 1);
-    if (jobs[j].x != jobs[0].x || (jobs[j].ldx ? jobs[j].ldx : ldx) != (jobs[0].ldx ? jobs[0].ldx : ldx))
-      return p;  // one activation matrix per launch
+// Shape plans of this thread's recent launches: the search tries every instantiated shape and split (about
+// 5 us of host time at K = 5632), and a program's calls repeat a few shapes.
+struct PlanKey {
+  size_t K, rows[kMaxJobsM], xld;
+  int batch, n_jobs, flags, qtype[kMaxJobsM];
+  bool operator==(const PlanKey& o) const {
+    return K == o.K && xld == o.xld && batch == o.batch && n_jobs == o.n_jobs && flags == o.flags &&
+           std::equal(rows, rows + kMaxJobsM, o.rows) && std::equal(qtype, qtype + kMaxJobsM, o.qtype);
   }
-  const size_t xld = jobs[0].ldx ? jobs[0].ldx : ldx;
-  if (reinterpret_cast<uintptr_t>(jobs[0].x) % 16 != 0 || xld % 4 != 0) return p;
-  p.nm = epi == kEpiSwiglu ? 2 : 1;
+};
+struct PlanMemo {
+  static constexpr int kEntries = 16;
+  PlanKey key[kEntries];
+  Plan plan[kEntries];
+  int used = 0, next = 0;
+  const Plan* find(const PlanKey& k) const {
+    for (int i = 0; i < used; ++i)
+      if (key[i] == k) return &plan[i];
+    return nullptr;
+  }
+  void put(const PlanKey& k, const Plan& p) {
+    key[next] = k;
+    plan[next] = p;
+    next = (next + 1) % kEntries;
+    used = std::min(used + 1, kEntries);
+  }
+};
+thread_local PlanMemo t_plans;
+
+// The part of plan_mfma that depends on a PlanKey only.
+Plan plan_shape(Plan p, const GemvJob* jobs, int n_jobs, int batch, size_t xld, size_t K, size_t wbytes, bool staged,
+                bool even_rt) {
   // decided by the count of 16-sequence tiles, so workspaces sized by tile counts hold for every batch
   const int padded = (batch + kSeqTile - 1) / kSeqTile * kSeqTile;
   double macs = 0.0;
@@ -1421,6 +1434,43 @@ Plan plan_mfma(const GemvJob* jobs, int n_jobs, int epi, int batch, size_t ldx, 
   return p;
 }
 
+
+// staged: the launch reads producer-staged tables (never the many-sequence kernel); even_rt: only shapes
+// whose workgroup rows are a multiple of 32 (outputs staged as tables).
+Plan plan_mfma(const GemvJob* jobs, int n_jobs, int epi, int batch, size_t ldx, bool staged = false,
+               bool even_rt = false) {
+  Plan p;
+  if (batch < 2 || n_jobs < 1 || n_jobs > kMaxJobsM) return p;
+  const size_t K = jobs[0].W->cols;
+  if (K % 32 != 0 || K > 65536) return p;
+  size_t wbytes = 0;
+  for (int j = 0; j < n_jobs; ++j) {
+    if (jobs[j].W->qtype != EF_QTYPE_Q4_0 && jobs[j].W->qtype != EF_QTYPE_Q8_0) return Plan{};
+    p.q4 = p.q4 || jobs[j].W->qtype == EF_QTYPE_Q4_0;
+    p.q8 = p.q8 || jobs[j].W->qtype == EF_QTYPE_Q8_0;
+    wbytes += jobs[j].W->rows * jobs[j].W->row_bytes * (jobs[j].W2 ? 2 : 1);
+    if (jobs[j].x != jobs[0].x || (jobs[j].ldx ? jobs[j].ldx : ldx) != (jobs[0].ldx ? jobs[0].ldx : ldx))
+      return p;  // one activation matrix per launch
+  }
+  const size_t xld = jobs[0].ldx ? jobs[0].ldx : ldx;
+  if (reinterpret_cast<uintptr_t>(jobs[0].x) % 16 != 0 || xld % 4 != 0) return p;
+  p.nm = epi == kEpiSwiglu ? 2 : 1;
+  PlanKey key{};
+  key.K = K;
+  key.batch = batch;
+  key.n_jobs = n_jobs;
+  key.flags = p.nm * 4 + (staged ? 2 : 0) + (even_rt ? 1 : 0);
+  for (int j = 0; j < n_jobs; ++j) {
+    key.rows[j] = jobs[j].W->rows;
+    key.qtype[j] = jobs[j].W->qtype;
+  }
+  key.xld = static_cast<size_t>(batch) * xld * 4 >= (size_t(1) << 32) ? xld : 0;  // decides only above 4 GiB
+  if (const Plan* kept = t_plans.find(key)) return *kept;
+  p = plan_shape(p, jobs, n_jobs, batch, xld, K, wbytes, staged, even_rt);
+  t_plans.put(key, p);
+  return p;
+}
+
 }  // namespace
 
 size_t tiled_bytes(const ef_hip_weight_s* w) {
@@ -1475,6 +1525,52 @@ size_t gemv_mfma_workspace_bytes(const GemvJob* jobs, int n_jobs, int epi, int b
 }
 
 
+namespace {
+// The workspace of calls on the library's own stream that bring none: kept from call to call (a
+// stream-ordered allocation and its release cost about 10 us of host time per call), grown by
+// stream-ordered calls, at most kKeepBytes, given back by ef_hip_shutdown.  A call holds the lock until
+// its launches are enqueued, so callers of several threads take turns, and the stream orders their uses.
+// Other streams and captured calls (whose graph could outlive the buffer) allocate as before.
+constexpr size_t kKeepBytes = size_t(256) << 20;
+std::mutex g_keep_mu;
+void* g_keep = nullptr;
+size_t g_keep_bytes = 0;
+
+// The kept workspace with at least `bytes` bytes (the caller holds g_keep_mu); null when the call has to
+// allocate its own.
+int kept_workspace(size_t bytes, hipStream_t stream, void** out) {
+  *out = nullptr;
+  if (stream != ctx().stream || bytes > kKeepBytes) return EF_HIP_OK;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  EFH_HIP(hipStreamIsCapturing(stream, &st));
+  if (st != hipStreamCaptureStatusNone) return EF_HIP_OK;
+  if (g_keep_bytes < bytes) {
+    size_t want = size_t(1) << 20;
+    while (want < bytes) want *= 2;
+    if (g_keep != nullptr) {
+      void* old = g_keep;
+      g_keep = nullptr;
+      g_keep_bytes = 0;
+      EFH_HIP(hipFreeAsync(old, stream));
+    }
+    EFH_HIP(hipMallocAsync(&g_keep, want, stream));
+    g_keep_bytes = want;
+  }
+  *out = g_keep;
+  return EF_HIP_OK;
+}
+}  // namespace
+
+int release_gemv_workspace(hipStream_t stream) {
+  std::lock_guard<std::mutex> lk(g_keep_mu);
+  if (g_keep == nullptr) return EF_HIP_OK;
+  void* old = g_keep;
+  g_keep = nullptr;
+  g_keep_bytes = 0;
+  EFH_HIP(hipFreeAsync(old, stream));
+  return EF_HIP_OK;
+}
+
 int launch_gemv_mfma(const GemvJob* jobs, int n_jobs, int epi, const float* norm_w, float eps, int batch, size_t ldx,
                      size_t ldy, void* ws, size_t ws_bytes, hipStream_t stream, bool* taken) {
   *taken = false;
@@ -1487,12 +1583,18 @@ int launch_gemv_mfma(const GemvJob* jobs, int n_jobs, int epi, const float* norm
   }
   const size_t K = jobs[0].W->cols;
   const size_t xld = jobs[0].ldx ? jobs[0].ldx : ldx;
-  // workspace: the caller's, else a stream-ordered allocation freed after the launches
+  // workspace: the caller's, else the kept one, else a stream-ordered allocation freed after the launches
   void* buf = ws;
   bool own = false;
+  std::unique_lock<std::mutex> keep_lock(g_keep_mu, std::defer_lock);
   if (buf == nullptr || ws_bytes < pl.bytes) {
-    EFH_HIP(hipMallocAsync(&buf, pl.bytes, stream));
-    own = true;
+    keep_lock.lock();
+    EFH_RC(kept_workspace(pl.bytes, stream, &buf));
+    if (buf == nullptr) {
+      keep_lock.unlock();
+      EFH_HIP(hipMallocAsync(&buf, pl.bytes, stream));
+      own = true;
+    }
   }
   uint8_t* base = static_cast<uint8_t*>(buf);
   uint8_t* t4 = pl.q4 ? base : nullptr;

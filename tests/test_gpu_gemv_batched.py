@@ -244,3 +244,37 @@ def test_many_sequence_kernel_swiglu_and_mixed_jobs(hip):
     for (W, _, y), w64 in zip(jobs, mats):
         err = np.abs(y.numpy()[:, :W.rows] - h @ w64.T) / np.maximum(np.abs(h) @ np.abs(w64).T, 1e-30)
         assert err.max() < REL_TOL
+
+
+def test_kept_workspace_is_shared_in_order(hip):
+    """Calls on the library's stream keep one workspace: calls that grow it, calls of other shapes between
+    them and calls from two threads give the bits of calls on a stream of their own (which allocate)."""
+    import threading
+    shapes = [(128, 1024, 5), (64, 2048, 40), (256, 5632, 64), (96, 4096, 300), (128, 1024, 5)]
+    work = []
+    for i, (rows, cols, batch) in enumerate(shapes):
+        W = hip.Weight(O.Q4_0, rows, cols, host=D.random_rows(O.Q4_0, rows, cols, seed=120 + i))
+        x = hip.DeviceArray.from_host(_batch_x(2000 + i, batch, cols))
+        work.append((W, x, batch))
+    s = hip.Stream()
+    want = []
+    for W, x, batch in work:
+        y = hip.DeviceArray((batch, W.rows))
+        hip.matvec(W, x, y, batch=batch, stream=s)
+        want.append(y.numpy(s))
+    outs = [[hip.DeviceArray((b, W.rows)) for W, _, b in work] for _ in range(2)]
+
+    def enqueue(k):
+        for _ in range(20):
+            for (W, x, batch), y in zip(work, outs[k]):
+                hip.matvec(W, x, y, batch=batch)
+
+    threads = [threading.Thread(target=enqueue, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    hip.sync()
+    for k in range(2):
+        for y, w in zip(outs[k], want):
+            assert np.array_equal(y.numpy().view(np.uint32), w.view(np.uint32))
