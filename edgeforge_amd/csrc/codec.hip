@@ -130,9 +130,10 @@ __device__ float q4_scale(const float (&x)[32], bool search) {
 // A workgroup packs kQuantBlocks consecutive blocks: their weights come in coalesced through LDS (rows of
 // 33 floats, so that the threads' reads fall in distinct banks) and their bytes leave through it the
 // same way.  Bound by vector issue: eight tries of 32 weights at seven instructions, four of them on
-// doubles (the reference's sequential double sums).  5632x2048 Q4_0 with the search: 54.3 us per call
-// with strided loads, codes kept per try and twice the instructions, 40.8 us so (1.3 TB/s).
-constexpr int kQuantBlocks = 256;
+// doubles (the reference's sequential double sums).  Q4_0 with the search, 5632x2048: 54.5 us per call
+// with strided loads, codes kept per try and twice the instructions, 39.8 us so (1.3 TB/s; 500x512
+// 14.5 -> 10.5); Q8_0 11.7 -> 10.9 (4.8 TB/s).  256 blocks per workgroup cost small matrices 0.7 to 2 us.
+constexpr int kQuantBlocks = 64;  // one wave: small matrices reach more CUs, and the tail is short
 
 template <bool Q4>
 __global__ __launch_bounds__(kQuantBlocks) void quantize_blocks_kernel(const float* __restrict__ w, long blocks,
@@ -155,8 +156,15 @@ __global__ __launch_bounds__(kQuantBlocks) void quantize_blocks_kernel(const flo
       p[2] = v[i].z;
       p[3] = v[i].w;
     }
-  } else {
-    for (int e = t; e < n * 32; e += kQuantBlocks) xs[(e >> 5) * kLd + (e & 31)] = src[e];
+  } else {  // the last blocks, or weights off a 16-byte boundary
+    float v[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) v[i] = t + kQuantBlocks * i < n * 32 ? src[t + kQuantBlocks * i] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const int e = t + kQuantBlocks * i;
+      xs[(e >> 5) * kLd + (e & 31)] = v[i];
+    }
   }
   __syncthreads();
   float x[32];
@@ -205,13 +213,10 @@ __global__ __launch_bounds__(kQuantBlocks) void quantize_blocks_kernel(const flo
   }
   __syncthreads();
   uint8_t* dst = out + g0 * kBytes;
-  const int bytes = n * kBytes;
-  if (n == kQuantBlocks && reinterpret_cast<uintptr_t>(dst) % 16 == 0) {
-    for (int i = t; i < bytes / 16; i += kQuantBlocks)
-      reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(xs)[i];
-  } else {
-    for (int i = t; i < bytes; i += kQuantBlocks) dst[i] = reinterpret_cast<const uint8_t*>(xs)[i];
-  }
+  const int bytes = n * kBytes, whole = reinterpret_cast<uintptr_t>(dst) % 16 == 0 ? bytes / 16 : 0;
+  for (int i = t; i < whole; i += kQuantBlocks)
+    reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(xs)[i];
+  for (int i = 16 * whole + t; i < bytes; i += kQuantBlocks) dst[i] = reinterpret_cast<const uint8_t*>(xs)[i];
 }
 
 __global__ void pack16_kernel(int qtype, const float* __restrict__ w, size_t n, uint16_t* __restrict__ out) {

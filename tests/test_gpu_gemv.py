@@ -209,9 +209,9 @@ def test_rows_f32_is_exact_dequantization(hip, qtype):
 
 
 @pytest.mark.parametrize("qtype", [O.Q4_0, O.Q8_0])
-@pytest.mark.parametrize("rows,cols,off", [(1, 32, 0), (3, 96, 0), (255, 32, 0), (257, 32, 0), (5, 4128, 1)])
+@pytest.mark.parametrize("rows,cols,off", [(1, 32, 0), (3, 96, 0), (63, 32, 0), (65, 32, 0), (257, 32, 0), (5, 4128, 1)])
 def test_quantizer_block_counts_and_alignment(hip, qtype, rows, cols, off):
-    """Block counts around a workgroup's 256 (one, partial, one more) and, with off, an input at a 4-byte
+    """Block counts around the workgroups (one, partial, one more) and, with off, an input at a 4-byte
     and an output at an odd address: bytes identical to the oracle, and none written past the end.
     Weights of every size the clamp meets: values whose codes overflow an int next to NaN blocks."""
     print(f"[case] quantizer qtype={qtype} {rows}x{cols} off={off}", flush=True)
