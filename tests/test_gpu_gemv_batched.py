@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from edgeforge_amd import _lib as L
 from tests import _data as D
 
 pytestmark = pytest.mark.gpu
@@ -214,6 +215,15 @@ def test_many_sequence_kernel_edges(hip, qtype, rows, cols, batch):
     hip.matvec_residual(W, dx, dy, batch=batch)
     # the same sums added to y: one more rounding of the result
     assert np.abs(dy.numpy() - (base + got)).max() <= 2.0 ** -23 * (np.abs(base) + np.abs(got)).max()
+    # rows of x and y further apart than their lengths: the same bits, and nothing between the rows of y
+    ldx, ldy = cols + 4, rows + 3
+    wide = np.zeros((batch, ldx), np.float32)
+    wide[:, :cols] = X
+    dx2, dy2 = hip.DeviceArray.from_host(wide), hip.DeviceArray.from_host(np.full((batch, ldy), 7.0, np.float32))
+    L.call("ef_hip_matvec", W.handle, dx2.ptr, dy2.ptr, batch, ldx, ldy, None)
+    got2 = dy2.numpy()
+    assert np.array_equal(got2[:, :rows].view(np.uint32), got.view(np.uint32))
+    assert (got2[:, rows:] == 7.0).all()
 
 
 def test_many_sequence_kernel_swiglu_and_mixed_jobs(hip):
