@@ -1084,15 +1084,15 @@ __global__ __launch_bounds__(kBatchThreads) void attention_batch_kernel(AttnArgs
 #pragma unroll
     for (int pt = 0; pt < 2; ++pt) {
       const bool cur = c0 + 16 * pt + m == pos;
-      f4n part[2] = {zero, zero};
+      f4n part[4] = {zero, zero, zero, zero};  // of 16 dims each
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          part[j / 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur ? kn[j][e] : k[pt][j][e], q[j][e], part[j / 2], 0, 0, 0);
+          part[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur ? kn[j][e] : k[pt][j][e], q[j][e], part[j], 0, 0, 0);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        sc[pt][r] = c0 + 16 * pt + 4 * g + r <= pos ? part[0][r] + part[1][r] : -INFINITY;
+        sc[pt][r] = c0 + 16 * pt + 4 * g + r <= pos ? (part[0][r] + part[1][r]) + (part[2][r] + part[3][r]) : -INFINITY;
     }
     if (next <= pos) fetch_k(next, pos);
     float cm = -INFINITY;
@@ -1227,7 +1227,7 @@ __global__ __launch_bounds__(kAttnThreads) void prefill_attention_kernel(Prefill
 // Scores, exponentials and p.v are FP32, the sum of a row's exponentials is double, as in
 // kern::attention_heads (src/kernels.cpp:77-92,153-174); a chunk's p.v is summed on its own and
 // added to the running one, each new maximum rescales the running sums, and 1 / sum is applied at the
-// end.  Scores have two partial sums and p.v one per chunk, so no chain of additions is long.
+// end.  Scores have four partial sums and p.v one per chunk, so no chain of additions is long.
 // Positions past a row's own take no part (score -inf, V rows past the block's last position zero); a
 // maximum of -inf subtracts 0, so a row whose first chunks are all -inf still sums the rest.
 //
@@ -1300,19 +1300,16 @@ __global__ __launch_bounds__(256) void prefill_mfma_kernel(PrefillArgs pa, int n
     f4n sc[4];
 #pragma unroll
     for (int pt = 0; pt < 4; ++pt) {
-      f4n part[2];  // two partial sums of 32 dims each
+      f4n part[4];  // four partial sums of 16 dims each
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        part[h] = f4n{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int j = 0; j < 4; ++j) {
+        const f4n k = *reinterpret_cast<const f4n*>(ks + (16 * pt + m) * kPfLd + 16 * j + 4 * g);
+        part[j] = f4n{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int j = 2 * h; j < 2 * h + 2; ++j) {
-          const f4n k = *reinterpret_cast<const f4n*>(ks + (16 * pt + m) * kPfLd + 16 * j + 4 * g);
-#pragma unroll
-          for (int s = 0; s < 4; ++s) part[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[s], q[j][s], part[h], 0, 0, 0);
-        }
+        for (int s = 0; s < 4; ++s) part[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[s], q[j][s], part[j], 0, 0, 0);
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sc[pt][r] = part[0][r] + part[1][r];
+      for (int r = 0; r < 4; ++r) sc[pt][r] = (part[0][r] + part[1][r]) + (part[2][r] + part[3][r]);
     }
     if (c0 + kPfChunk > pfirst) {  // a chunk that some row of the workgroup does not see whole
       const int last = prow - c0 - 4 * g;  // position 16 pt + 4 g + r of the chunk takes part when 16 pt + r <= last
