@@ -1008,7 +1008,8 @@ __global__ __launch_bounds__(kSplitThreads) void attention_combine_kernel(AttnAr
 // straight into operands of v_mfma_f32_16x16x4_f32 (prefill_mfma_kernel's layouts and sums, the pairs
 // being the group's heads; columns past them idle).  A chunk's K registers are refilled once its
 // scores are formed and its V registers once they are used, so each wave keeps a chunk in flight.
-// The waves' sums are combined through LDS in wave order.
+// The waves' sums are combined through LDS in wave order, by what their exponentials were formed against
+// (the rounded maximum times c2), as the rescaling at each new maximum is (prefill_mfma_kernel).
 //
 // Bound by reading the cache, 2 x 256 bytes per position and workgroup: 30.0 us per layer at position 900
 // of 64 sequences x 4 groups (118 MB, 3.9 TB/s; a large copy reaches 5.1), where the KV-group kernel,
@@ -1104,11 +1105,11 @@ __global__ __launch_bounds__(kBatchThreads) void attention_batch_kernel(AttnArgs
     cm = fmaxf(cm, __shfl_xor(cm, 32, kWave));
     float al = 1.0f;
     if (__any(cm > mx)) {
-      const float nm = fmaxf(mx, cm);
-      sub = nm == -INFINITY ? 0.0f : nm * c2;
-      al = __builtin_amdgcn_exp2f(fmaf(mx, c2, -sub));
+      const float nm = fmaxf(mx, cm), ns = nm == -INFINITY ? 0.0f : nm * c2;
+      al = mx == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(sub - ns);
       l *= static_cast<double>(al);
       mx = nm;
+      sub = ns;
     }
     f4n oc[4] = {zero, zero, zero, zero};  // the chunk's own p.v
 #pragma unroll
@@ -1137,7 +1138,7 @@ __global__ __launch_bounds__(kBatchThreads) void attention_batch_kernel(AttnArgs
   for (int r = 0; r < 4; ++r)
     *reinterpret_cast<f4n*>(so[wave] + m * kBatchLd + 16 * g + 4 * r) = f4n{o[0][r], o[1][r], o[2][r], o[3][r]};
   if (g == 0) {
-    sm[wave][m] = mx;
+    sm[wave][m] = mx == -INFINITY ? -INFINITY : sub;
     sl[wave][m] = l;
   }
   __syncthreads();
@@ -1147,12 +1148,12 @@ __global__ __launch_bounds__(kBatchThreads) void attention_batch_kernel(AttnArgs
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < kBatchWaves; ++w) M = fmaxf(M, sm[w][hh]);
-    const float ms = M == -INFINITY ? 0.0f : M * c2;
+    const float ms = M == -INFINITY ? 0.0f : M;
     float acc = 0.0f;
     double L = 0.0;
 #pragma unroll
     for (int w = 0; w < kBatchWaves; ++w) {
-      const float f = __builtin_amdgcn_exp2f(fmaf(sm[w][hh], c2, -ms));  // 0 for a wave without a position
+      const float f = __builtin_amdgcn_exp2f(sm[w][hh] - ms);  // 0 for a wave without a position
       acc = fmaf(so[w][hh * kBatchLd + d], f, acc);
       L += sl[w][hh] * static_cast<double>(f);
     }
@@ -1228,6 +1229,10 @@ __global__ __launch_bounds__(kAttnThreads) void prefill_attention_kernel(Prefill
 // kern::attention_heads (src/kernels.cpp:77-92,153-174); a chunk's p.v is summed on its own and
 // added to the running one, each new maximum rescales the running sums, and 1 / sum is applied at the
 // end.  Scores have four partial sums and p.v one per chunk, so no chain of additions is long.
+// Exponentials are formed against sub, the rounded maximum times c2, and the rescaling is by the
+// difference of the two sub: exactly 1 for a pair whose maximum stays while another of its wave rises, and
+// consistent with the terms already summed however large the scores' common part is (1999 positions with
+// scores around 40: at most 1.5e-7 from float64; rescaling by the unrounded maximum gave 8.2e-6).
 // Positions past a row's own take no part (score -inf, V rows past the block's last position zero); a
 // maximum of -inf subtracts 0, so a row whose first chunks are all -inf still sums the rest.
 //
@@ -1328,11 +1333,11 @@ __global__ __launch_bounds__(256) void prefill_mfma_kernel(PrefillArgs pa, int n
     cm = fmaxf(cm, __shfl_xor(cm, 32, kWave));
     float al = 1.0f;
     if (__any(cm > mx)) {
-      const float nm = fmaxf(mx, cm);
-      sub = nm == -INFINITY ? 0.0f : nm * c2;
-      al = __builtin_amdgcn_exp2f(fmaf(mx, c2, -sub));
+      const float nm = fmaxf(mx, cm), ns = nm == -INFINITY ? 0.0f : nm * c2;
+      al = mx == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(sub - ns);
       l *= static_cast<double>(al);
       mx = nm;
+      sub = ns;
     }
     f4n oc[4];  // the chunk's own p.v
 #pragma unroll
