@@ -1234,7 +1234,8 @@ __global__ __launch_bounds__(kAttnThreads) void prefill_attention_kernel(Prefill
 // consistent with the terms already summed however large the scores' common part is (1999 positions with
 // scores around 40: at most 1.5e-7 from float64; rescaling by the unrounded maximum gave 8.2e-6).
 // Positions past a row's own take no part (score -inf, V rows past the block's last position zero); a
-// maximum of -inf subtracts 0, so a row whose first chunks are all -inf still sums the rest.
+// maximum of -inf subtracts 0, so a row whose first chunks are all -inf still sums the rest.  Chunks on the
+// diagonal whose sums come out infinite or NaN are summed again without what the row does not see.
 //
 // Bound by the FP32 matrix rate (151 TFLOP/s for a large library product on this GPU: 109 us for the
 // causal half of 1999 positions x 32 heads): 186 us, 31 us at 510 positions.  The vector-ALU
@@ -1246,7 +1247,7 @@ constexpr int kPfPairs = 64, kPfChunk = 64, kPfLd = 68;
 // 280 / 283, 1 x 64 (32) 332 / 318, 4 x 23 (48) 434 / 421, 64 x 23 2636 / 2257.
 constexpr int kPfMfmaFrom = 128, kPfMfmaWorkgroups = 32;
 
-__global__ __launch_bounds__(256) void prefill_mfma_kernel(PrefillArgs pa, int nseq, int cus) {
+__global__ __launch_bounds__(256, 3) void prefill_mfma_kernel(PrefillArgs pa, int nseq, int cus) {
   const AttnArgs& a = pa.a;
   __shared__ float ks[kPfChunk * kPfLd], vs[kPfChunk * kPfLd];
   const int t = threadIdx.x, wave = t / kWave, lane = t & (kWave - 1), m = lane & 15, g = lane >> 4;
@@ -1352,6 +1353,36 @@ __global__ __launch_bounds__(256) void prefill_mfma_kernel(PrefillArgs pa, int n
 #pragma unroll
         for (int d = 0; d < 4; ++d) oc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[d], e, oc[d], 0, 0, 0);
       }
+    if (c0 + kPfChunk > pfirst) {
+      // A product with a position that the row does not see is 0 V: an infinite or NaN V must not reach the
+      // row, so such a chunk is summed again over each row's own positions.
+      bool bad = false;
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bad = bad || !(fabsf(oc[d][r]) < INFINITY);
+      if (__any(bad)) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) oc[d] = f4n{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float own = __builtin_amdgcn_exp2f(fmaf(sc[pt][r], c2, -sub));
+#pragma unroll 1
+            for (int gp = 0; gp < 4; ++gp) {  // position 16 pt + 4 gp + r, whose exponential lane 16 gp + m has
+              const float e = __shfl(own, 16 * gp + m, kWave);
+              if (c0 + 16 * pt + 4 * gp + r <= prow) {
+                const float* vp = vs + (16 * pt + 4 * gp + r) * kPfLd + 16 * g;
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                  for (int d = 0; d < 4; ++d) oc[d][u] = fmaf(vp[4 * u + d], e, oc[d][u]);
+              }
+            }
+          }
+      }
+    }
 #pragma unroll
     for (int d = 0; d < 4; ++d)
 #pragma unroll

@@ -10,6 +10,7 @@ import os
 import numpy as np
 import pytest
 
+from edgeforge_amd import _lib as L
 from edgeforge_amd.model import Config, DeviceModel, Engine
 from oracle.model import OracleModel
 from tests import _data as D
@@ -145,3 +146,28 @@ def test_matrix_core_prefill_attention_edges(hip, monkeypatch, H, KV, B, n, rows
         got[kind] = eng.logits().copy()
         eng.close()
     assert _err(got["tiled"], got["rows"]) < 1e-5
+
+
+@pytest.mark.parametrize("cfg,n,bad", [(TILE4, 40, 30), (TILE, 200, 150), (TILE4, 200, 64)])
+def test_prefill_attention_keeps_a_nan_to_its_later_positions(hip, monkeypatch, cfg, n, bad):
+    """A NaN embedding at one position: the positions before it keep the bits they have without it (they
+    share workgroups and chunks of V rows with it), that position and the later ones are NaN."""
+    print(f"[case] prefill with a NaN at {bad} of {n}, H={cfg.H} KV={cfg.KV}", flush=True)
+    monkeypatch.setenv("EF_HIP_PREFILL_ATTENTION", "tiled")
+    dm = DeviceModel.synthetic(cfg, seed=75)
+    nan_id = cfg.V - 1
+    row = np.full(cfg.D, 0x7FC0, np.uint16)  # BF16 NaN
+    L.call("ef_hip_memcpy_h2d", dm.packed["embed"].ptr + nan_id * row.nbytes, row.ctypes.data, row.nbytes, None)
+    ids = D.rng(76).integers(0, nan_id, size=n).astype(np.int32)
+    eng = Engine(dm, max_seq=n)
+    out = {}
+    for kind in ("clean", "nan"):
+        if kind == "nan":
+            ids[bad] = nan_id
+        logits = hip.DeviceArray((n - 1, cfg.V))
+        eng.score(ids, 0, logits)
+        out[kind] = logits.numpy()
+    eng.close()
+    assert np.isfinite(out["clean"]).all()
+    assert np.array_equal(out["nan"][:bad].view(np.uint32), out["clean"][:bad].view(np.uint32))
+    assert np.isnan(out["nan"][bad:]).all()
