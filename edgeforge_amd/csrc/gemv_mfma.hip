@@ -47,6 +47,7 @@
 
 #include "afrag.h"
 #include "gemv.h"
+#include "kept.h"
 #include "qfrag.h"
 
 namespace efh {
@@ -1531,10 +1532,10 @@ namespace {
 // stream-ordered calls, at most kKeepBytes, given back by ef_hip_shutdown.  A call holds the lock until
 // its launches are enqueued, so callers of several threads take turns, and the stream orders their uses.
 // Other streams and captured calls (whose graph could outlive the buffer) allocate as before.
+// A call whose rounded size cannot be had asks for its own size, there or for itself.
 constexpr size_t kKeepBytes = size_t(256) << 20;
 std::mutex g_keep_mu;
-void* g_keep = nullptr;
-size_t g_keep_bytes = 0;
+KeptBuffer g_keep;
 
 // The kept workspace with at least `bytes` bytes (the caller holds g_keep_mu); null when the call has to
 // allocate its own.
@@ -1544,29 +1545,26 @@ int kept_workspace(size_t bytes, hipStream_t stream, void** out) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   EFH_HIP(hipStreamIsCapturing(stream, &st));
   if (st != hipStreamCaptureStatusNone) return EF_HIP_OK;
-  if (g_keep_bytes < bytes) {
-    size_t want = size_t(1) << 20;
-    while (want < bytes) want *= 2;
-    if (g_keep != nullptr) {
-      void* old = g_keep;
-      g_keep = nullptr;
-      g_keep_bytes = 0;
-      EFH_HIP(hipFreeAsync(old, stream));
-    }
-    EFH_HIP(hipMallocAsync(&g_keep, want, stream));
-    g_keep_bytes = want;
-  }
-  *out = g_keep;
+  hipError_t freed = hipSuccess;
+  *out = kept_at_least(
+      g_keep, bytes,
+      [&](size_t n) -> void* {
+        void* p = nullptr;
+        if (hipMallocAsync(&p, n, stream) == hipSuccess) return p;
+        (void)hipGetLastError();  // not for the launches that follow
+        return nullptr;
+      },
+      [&](void* p) { freed = hipFreeAsync(p, stream); });
+  EFH_HIP(freed);
   return EF_HIP_OK;
 }
 }  // namespace
 
 int release_gemv_workspace(hipStream_t stream) {
   std::lock_guard<std::mutex> lk(g_keep_mu);
-  if (g_keep == nullptr) return EF_HIP_OK;
-  void* old = g_keep;
-  g_keep = nullptr;
-  g_keep_bytes = 0;
+  if (g_keep.p == nullptr) return EF_HIP_OK;
+  void* old = g_keep.p;
+  g_keep = KeptBuffer{};
   EFH_HIP(hipFreeAsync(old, stream));
   return EF_HIP_OK;
 }
