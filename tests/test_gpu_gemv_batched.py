@@ -7,6 +7,10 @@ batches that are not a multiple of the 16-sequence tile, many tiles in one launc
 sequences (several launches), row counts that leave a partial workgroup, Q8_0, a K split (K = 5632
 at B = 64) and mixed-type launches; epilogues and the fused RMSNorm are checked against the oracle's separate operations.
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -16,6 +20,7 @@ from tests import _data as D
 
 pytestmark = pytest.mark.gpu
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ABS_TOL = 1e-4
 REL_TOL = 1e-5
 
@@ -257,8 +262,8 @@ def test_many_sequence_kernel_swiglu_and_mixed_jobs(hip):
 
 
 def test_kept_workspace_is_shared_in_order(hip):
-    """Calls on the library's stream keep one workspace: calls that grow it, calls of other shapes between
-    them and calls from two threads give the bits of calls on a stream of their own (which allocate)."""
+    """Calls on the library's stream keep one workspace: calls of different shapes in turn and from two
+    threads give the bits of calls on a stream of their own (which allocate)."""
     import threading
     shapes = [(128, 1024, 5), (64, 2048, 40), (256, 5632, 64), (96, 4096, 300), (128, 1024, 5)]
     work = []
@@ -288,3 +293,36 @@ def test_kept_workspace_is_shared_in_order(hip):
     for k in range(2):
         for y, w in zip(outs[k], want):
             assert np.array_equal(y.numpy().view(np.uint32), w.view(np.uint32))
+
+
+def _grow_kept_workspace():
+    """(In a process of its own, where nothing is kept yet.)  Workspaces of 0.1 to 70 MB, each call one that
+    replaces the kept buffer while the launches that use the old one are still queued."""
+    from edgeforge_amd import hip
+    hip.init(0)
+    work = []
+    for i, (rows, cols, batch) in enumerate([(64, 1024, 5), (64, 2048, 200), (96, 4096, 300), (64, 5632, 600),
+                                             (64, 5632, 1000), (64, 14336, 1000)]):
+        W = hip.Weight(O.Q4_0, rows, cols, host=D.random_rows(O.Q4_0, rows, cols, seed=140 + i))
+        x = hip.DeviceArray.from_host(_batch_x(2100 + i, batch, cols))
+        work.append((W, x, batch))
+    s = hip.Stream()
+    want = []
+    for W, x, batch in work:  # also makes the tile-order copies
+        y = hip.DeviceArray((batch, W.rows))
+        hip.matvec(W, x, y, batch=batch, stream=s)
+        want.append(y.numpy(s))
+    outs = [(i, hip.DeviceArray((batch, W.rows))) for i, (W, x, batch) in enumerate(work) for _ in range(30)]
+    for i, y in outs:  # queued behind each other; the first of each shape replaces the kept workspace
+        hip.matvec(work[i][0], work[i][1], y, batch=work[i][2])
+    hip.sync()
+    for i, y in outs:
+        assert np.array_equal(y.numpy().view(np.uint32), want[i].view(np.uint32)), i
+    print("grown", flush=True)
+
+
+def test_kept_workspace_grows_under_queued_launches():
+    print("[case] kept workspace growth in a process of its own", flush=True)
+    r = subprocess.run([sys.executable, "-c", "from tests import test_gpu_gemv_batched as t; t._grow_kept_workspace()"],
+                       cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "grown" in r.stdout, (r.returncode, r.stdout, r.stderr)
