@@ -1003,21 +1003,29 @@ __global__ __launch_bounds__(kSplitThreads) void attention_combine_kernel(AttnAr
 }
 
 // Decode attention of a large batch (hd = 64, at most 16 query heads per KV head): one workgroup per
-// (KV group, sequence), as attention_group_kernel, but one pass with a running
-// maximum and no staging: the eight waves take 32-position chunks in turn and read their K and V rows
-// straight into operands of v_mfma_f32_16x16x4_f32 (prefill_mfma_kernel's layouts and sums, the pairs
-// being the group's heads; columns past them idle).  A chunk's K registers are refilled once its
-// scores are formed and its V registers once they are used, so each wave keeps a chunk in flight.
-// The waves' sums are combined through LDS in wave order, by what their exponentials were formed against
-// (the rounded maximum times c2), as the rescaling at each new maximum is (prefill_mfma_kernel).
+// (KV group, sequence), as attention_group_kernel, but one pass with a running maximum and no staging:
+// its waves take 32-position chunks in turn and read their K and V rows straight into operands of
+// v_mfma_f32_16x16x4_f32 (prefill_mfma_kernel's layouts and sums, the pairs being the group's heads; columns
+// past them idle).  A chunk's K registers are refilled once its scores are formed and its V registers
+// once they are used, so each wave keeps a chunk in flight.  The waves' sums are combined through LDS in
+// wave order, by what their exponentials were formed against (the rounded maximum times c2), as the
+// rescaling at each new maximum is (prefill_mfma_kernel).
 //
 // Bound by reading the cache, 2 x 256 bytes per position and workgroup: 30.0 us per layer at position 900
-// of 64 sequences x 4 groups (118 MB, 3.9 TB/s; a large copy reaches 5.1), where the KV-group kernel,
-// which stages each 64-position chunk between barriers in two passes, took 77.7; 50.9 / 153.8 at 1900,
-// 8.3 / 12.2 at 100, 7.4 / 7.8 at 63.
-constexpr int kBatchThreads = 512, kBatchWaves = kBatchThreads / kWave, kBatchChunk = 32, kBatchHeads = 16, kBatchLd = 68;
+// of 64 sequences x 4 groups in a four-layer engine (118 MB, 3.9 TB/s; a large copy reaches 5.1), where the
+// KV-group kernel, which stages each 64-position chunk between barriers in two passes, took 77.7.  In a
+// one-layer engine, this / KV-group kernel, us at positions 1900, 900, 200, 63, 8: 256 workgroups 42.5 / 142.2,
+// 23.7 / 65.6, 9.7 / 19.8, 6.9 / 8.2, 6.9 / 6.9.
+//
+// A CU holds eight of its waves.  Up to one workgroup per CU has eight waves, up to two four, and more
+// two, so that the launch is one round as far as it can be: 1024 workgroups of 4 eight-head groups 99.2 / 297.0 at 900,
+// 13.4 / 30.3 at 63, of 16 two-head groups 85.7 / 145.9 and 10.3 / 16.1.  With eight waves always, all requesting their
+// first chunk, a step of the latter took 17 us longer than with the KV-group kernel at position 8.
+constexpr int kBatchChunk = 32, kBatchHeads = 16, kBatchLd = 68, kBatchEager = 2;
 
-__global__ __launch_bounds__(kBatchThreads) void attention_batch_kernel(AttnArgs a) {
+template <int kBatchWaves>
+__global__ __launch_bounds__(kBatchWaves * kWave) void attention_batch_kernel(AttnArgs a) {
+  constexpr int kBatchThreads = kBatchWaves * kWave;
   __shared__ float so[kBatchWaves][kBatchHeads * kBatchLd];
   __shared__ float sm[kBatchWaves][kBatchHeads];
   __shared__ double sl[kBatchWaves][kBatchHeads];
@@ -1042,9 +1050,13 @@ __global__ __launch_bounds__(kBatchThreads) void attention_batch_kernel(AttnArgs
       for (int r = 0; r < 4; ++r)
         v[pt][r] = *reinterpret_cast<const f4n*>(vc + static_cast<long>(min(c0 + 16 * pt + 4 * g + r, lim)) * kvd + 4 * m);
   };
-  // the first chunk is requested before the position is known (every row of the cache is in bounds)
-  fetch_k(wave * kBatchChunk, a.max_seq - 1);
-  fetch_v(wave * kBatchChunk, a.max_seq - 1);
+  // the first chunks of kBatchEager waves (64 positions, as the KV-group kernel) are requested before the position
+  // is known (every row of the cache is in bounds), the other waves' once it is: a short cache does not have them
+  const int first = wave * kBatchChunk;
+  if (wave < kBatchEager) {
+    fetch_k(first, a.max_seq - 1);
+    fetch_v(first, a.max_seq - 1);
+  }
   // RoPE in the operands' layout: dims i = 16 j + 4 g + s and i + 32 are in the same lane
   f4n q[4], kn[4];
   const float* qp = a.q + static_cast<long>(b) * a.ldq + (kv * hpg + min(m, hpg - 1)) * 64 + 4 * g;
@@ -1065,6 +1077,10 @@ __global__ __launch_bounds__(kBatchThreads) void attention_batch_kernel(AttnArgs
     }
   }
   const int pos = *a.pos_dev;
+  if (wave >= kBatchEager && first <= pos) {
+    fetch_k(first, pos);
+    fetch_v(first, pos);
+  }
   if (wave == 0) {  // k / v at pos for later steps
     float* kw = a.kcache + seq0 + static_cast<long>(pos) * kvd;
     float* vw = a.vcache + seq0 + static_cast<long>(pos) * kvd;
@@ -1574,11 +1590,18 @@ int launch_attention(const AttnArgs& a, int batch, hipStream_t s) {
   const size_t lim = std::max<size_t>(ctx().lds_per_block, 65536);
   const int cus = ctx().cu_count > 0 ? ctx().cu_count : 256;
   const int choice = attention_choice();
-  // the KV-group kernel's launches at hd = 64 (unless a kernel is forced): the matrix-core pass, faster at
-  // every position measured
+  // the KV-group kernel's launches at hd = 64 (unless a kernel is forced): the matrix-core pass, as fast at
+  // position 8 and faster from there on for every geometry measured (2, 4 and 8 heads per group, 128 to 1024 workgroups)
   if (choice == 0 && a.hd == 64 && a.rope_now != nullptr && a.ldq % 4 == 0 && a.H / a.KV <= kBatchHeads &&
       attention_uses_group(a, batch)) {
-    hipLaunchKernelGGL(attention_batch_kernel, dim3(a.KV, batch), dim3(kBatchThreads), 0, s, a);
+    const long wgs = static_cast<long>(a.KV) * batch;
+    if (wgs > 2 * cus) {
+      hipLaunchKernelGGL(attention_batch_kernel<2>, dim3(a.KV, batch), dim3(2 * kWave), 0, s, a);
+    } else if (wgs > cus) {
+      hipLaunchKernelGGL(attention_batch_kernel<4>, dim3(a.KV, batch), dim3(4 * kWave), 0, s, a);
+    } else {
+      hipLaunchKernelGGL(attention_batch_kernel<8>, dim3(a.KV, batch), dim3(8 * kWave), 0, s, a);
+    }
     EFH_HIP(hipGetLastError());
     return EF_HIP_OK;
   }

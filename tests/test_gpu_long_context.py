@@ -109,7 +109,11 @@ def test_position_split_equals_single_pass_within_tolerance(hip, B, monkeypatch)
         assert _logit_err(out["split"][1][k][0], want_logits[k]) < 1e-4, k
 
 
-@pytest.mark.parametrize("H,KV,B", [(4, 2, 64), (8, 1, 130)])
+@pytest.mark.parametrize("H,KV,B", [
+    (4, 2, 64), (8, 1, 130),  # eight waves per workgroup
+    (4, 2, 200),              # more workgroups than CUs: four
+    (4, 2, 300), (16, 1, 600),  # more than two per CU: two waves; 16 heads fill the operand's columns
+])
 def test_large_batch_attention(hip, monkeypatch, H, KV, B):
     """A large batch's steps run one matrix-core pass over the cache: its logits against the KV-group
     kernel's within 1e-5 relative (FP32 sums in another order, as the position split above), at the
