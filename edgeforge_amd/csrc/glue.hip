@@ -1260,7 +1260,13 @@ constexpr int kPfPairs = 64, kPfChunk = 64, kPfLd = 68;
 // The kernel runs from 128 positions per sequence, or from 32 workgroups: below that the one
 // workgroup per (head, row) kernel fills more of the GPU.  Four layers, 32 heads over 4 KV heads,
 // us per prefill, rows kernel / this one: 1 x 8 positions (4 workgroups) 254 / 262, 1 x 23 (12)
-// 280 / 283, 1 x 64 (32) 332 / 318, 4 x 23 (48) 434 / 421, 64 x 23 2636 / 2257.
+// 280 / 283, 1 x 64 (32) 332 / 318, 4 x 23 (48) 434 / 421, 64 x 23 2636 / 2257.  Few pairs in a workgroup
+// (one query head per KV head, a short continuation) do not change that, nor a long prefix: one layer, 32 heads
+// over 32 KV heads, one position of one sequence (32 workgroups of one pair) 69 / 71 from position 0,
+// 96 / 93 from 500, 211 / 175 from 2000, 714 / 492 from 8000; two positions of 32 sequences (1024 of two) 108 / 109
+// from 0, 205 / 170 from 500.  Only workgroups of a single pair that do not fit the CUs at once are
+// left to the rows kernel: one position of 32 sequences (1024) 89 / 94 from 0, 147 / 154 from 500, of 16 (512) 85 / 87 and
+// 128 / 118.
 constexpr int kPfMfmaFrom = 128, kPfMfmaWorkgroups = 32;
 
 __global__ __launch_bounds__(256, 3) void prefill_mfma_kernel(PrefillArgs pa, int nseq, int cus) {
@@ -1279,6 +1285,9 @@ __global__ __launch_bounds__(256, 3) void prefill_mfma_kernel(PrefillArgs pa, in
   const int kv = id % a.KV, b = id / a.KV % nseq, i0 = (nb - 1 - id / a.KV / nseq) * rpb;
   const int pair = 16 * wave + m, il = pair / hpg, hh = pair - il * hpg, i = i0 + il;
   const bool active = il < rpb && i < pa.n;
+  // waves without a pair (the last rows of a sequence, few rows of few heads) only stage
+  const int il0 = __builtin_amdgcn_readfirstlane(16 * wave / hpg);
+  const bool busy = il0 < rpb && i0 + il0 < pa.n;
   const int pos0 = *a.pos_dev;
   const int prow = pos0 + i, pfirst = pos0 + i0, plast = pos0 + min(i0 + rpb, pa.n) - 1;
   const long row = static_cast<long>(b) * pa.n + (active ? i : i0);
@@ -1319,6 +1328,10 @@ __global__ __launch_bounds__(256, 3) void prefill_mfma_kernel(PrefillArgs pa, in
     }
     __syncthreads();
     if (c0 + kPfChunk <= plast) fetch(c0 + kPfChunk);
+    if (!busy) {
+      __syncthreads();
+      continue;
+    }
     f4n sc[4];
 #pragma unroll
     for (int pt = 0; pt < 4; ++pt) {
@@ -1510,10 +1523,12 @@ int launch_prefill_attention(const PrefillArgs& a, int rows, hipStream_t s) {
   const bool force_rows = forced != nullptr && std::strcmp(forced, "rows") == 0;
   const bool force_tiled = forced != nullptr && std::strcmp(forced, "tiled") == 0;
   const int rpb = tiled_ok ? kPfPairs / hpg : 1, nb = (a.n + rpb - 1) / rpb, nseq = rows / a.n;
-  const bool enough = a.n >= kPfMfmaFrom || static_cast<long>(nseq) * nb * a.a.KV >= kPfMfmaWorkgroups;
+  const long wgs = static_cast<long>(nseq) * nb * a.a.KV;
+  const bool single = std::min(a.n, rpb) * hpg == 1 && wgs > 2L * std::max(1, ctx().cu_count);
+  const bool enough = a.n >= kPfMfmaFrom || (wgs >= kPfMfmaWorkgroups && !single);
   if (tiled_ok && !force_rows && (force_tiled || enough)) {
     EFH_CHECK(rows % a.n == 0, "prefill attention: rows must be sequences x positions");
-    hipLaunchKernelGGL(prefill_mfma_kernel, dim3(static_cast<unsigned>(nseq) * nb * a.a.KV), dim3(256), 0, s, a, nseq,
+    hipLaunchKernelGGL(prefill_mfma_kernel, dim3(static_cast<unsigned>(wgs)), dim3(256), 0, s, a, nseq,
                        std::max(1, ctx().cu_count));
     EFH_HIP(hipGetLastError());
     return EF_HIP_OK;

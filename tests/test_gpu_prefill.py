@@ -128,6 +128,8 @@ def test_tiled_prefill_attention_matches_rows_kernel_and_oracle(hip, monkeypatch
     (3, 1, 2, 65, 0),     # 21 rows x 3 heads (63 of 64 pairs), a one-position second chunk
     (16, 1, 1, 127, 60),  # 4 rows per workgroup, launches of 60, 60 and 7 positions
     (8, 4, 3, 1, 0),      # one position per sequence
+    (4, 4, 2, 17, 0),     # one head per KV head: a wave of 16 pairs, one of a single pair, two without
+    (2, 2, 300, 1, 0),    # 600 workgroups of a single pair
 ])
 def test_matrix_core_prefill_attention_edges(hip, monkeypatch, H, KV, B, n, rows):
     """The matrix-core prefill attention against the per-(head, row) kernel at the edges of its
@@ -139,13 +141,14 @@ def test_matrix_core_prefill_attention_edges(hip, monkeypatch, H, KV, B, n, rows
     dm = DeviceModel.synthetic(cfg, seed=80 + H)
     prompts = D.rng(81 + n).integers(0, cfg.V, size=(B, n)).astype(np.int32)
     got = {}
-    for kind in ("tiled", "rows"):
+    for kind in ("tiled", "rows", "auto"):
         monkeypatch.setenv("EF_HIP_PREFILL_ATTENTION", kind)
         eng = Engine(dm, max_seq=n + 1, batch=B)
         eng.prefill(prompts, 0)
         got[kind] = eng.logits().copy()
         eng.close()
     assert _err(got["tiled"], got["rows"]) < 1e-5
+    assert any(np.array_equal(got["auto"].view(np.uint32), got[k].view(np.uint32)) for k in ("tiled", "rows"))
 
 
 @pytest.mark.parametrize("cfg,n,bad", [(TILE4, 40, 30), (TILE, 200, 150), (TILE4, 200, 64)])
