@@ -1242,6 +1242,7 @@ struct Plan {
   size_t tab = 0, part_off = 0, bytes = 0, lds = 0;
   double cost = 0.0;
   bool rows = false;  // the many-sequence kernel (plan_rows per launch)
+  int rows_ns = 0, rows_kw = 0;  // its shape, where EF_HIP_GEMV_ROWS names one
 };
 
 int groups_for(const GemvJob* jobs, int n_jobs, int rows_wg) {
@@ -1275,12 +1276,19 @@ double shape_cost(int rt, int nm, int ns, int sg, int groups, int S, int bps, si
 }
 
 
-// The many-sequence kernel's launches: at most kRowsMax sequences, from kRowsFrom sequences and
-// kRowsMacs multiply-adds on (weight rows x matrices x sequences x K).  Below that its workgroups leave
-// CUs idle and the split-K kernel is the faster one; us per call, split-K / this one: 2048x2048 Q4_0
+// The many-sequence kernel's launches: at most kRowsMax sequences, from kRowsFrom sequences (after rounding up
+// to a tile) and kRowsMacs multiply-adds on (weight rows x matrices x sequences x K).  Below that its workgroups
+// leave CUs idle and the split-K kernel is the faster one; us per call, split-K / this one: 2048x2048 Q4_0
 // 500 sequences (2.1G) 28 / 33, 2048x5632 200 (2.3G) 37 / 39; SwiGLU 5632x2048 200 (4.6G) 52 / 47, 500
 // 80 / 73, 1500 214 / 184, 2048x5632 500 (5.8G) 62 / 57, 1024 109 / 90, 2048x2048 1500 (6.3G) 71 / 56,
 // Q8_0 32000x2048 200 (13G) 122 / 87, 510 228 / 164.
+// Above it only where the estimated time is not above the split-K kernel's: few rows, a long K, or a K whose
+// count of blocks is odd (no K share) leave CUs idle at more multiply-adds too; split-K / this one:
+// 512x14336 480 sequences 90 / 108, 1024x11264 304 55 / 71, 1000x4000 1024 49 / 93, 4096x4000 219 38 / 81,
+// 2048x5632 320 39 / 48 and 500 57 / 53.  kRowsShapes' times are of full launches; over 1621 shapes launches at the
+// line took 0.88, 0.73 and 0.6 of them with 1, 2 and 4 K shares.  With these, 28 of the shapes are more than 3%
+// slower than with the split-K kernel (one by 18%, the rest by at most 12%), against 151 (by up to 115%) from the
+// multiply-adds alone, and 7 are more than 3% slower than with this kernel (by at most 12%).
 constexpr int kRowsMax = 4096, kRowsFrom = 128;
 constexpr double kRowsMacs = 3.5e9;
 int rows_tiles(int rows) { return ((rows + kSeqTile - 1) / kSeqTile + 11) / 12 * 12; }  // a multiple of every NS
@@ -1298,6 +1306,7 @@ constexpr RowsShape kRowsShapes[] = {{4, 1, 0.66f, 1.03f}, {3, 1, 0.59f, 0.88f},
 struct RowsPlan {
   int NS = 0, KW = 1, groups = 0, sgs = 0;
   size_t lds = 0;
+  double cost = 0.0;  // us
 };
 
 template <int NM>
@@ -1309,25 +1318,31 @@ void* pick_rows(int ns, int kw) {
                  : (ns == 3 ? kf(&gemv_rows_kernel<NM, 3, 2>) : kf(&gemv_rows_kernel<NM, 2, 2>));
 }
 
-// The shape of the least estimated time for `rows` sequences: workgroups are dealt to the CUs evenly,
-// two to a CU at a time when their LDS allows it, plus 8 us per pair for its ends.
-RowsPlan plan_rows(const GemvJob* jobs, int n_jobs, int nm, int rows, bool q8) {
+// EF_HIP_GEMV_ROWS=ns,kw (tests): the many-sequence kernel in that shape wherever it can run; 0,0: never.
+// Read where a thread plans a launch for the first time (PlanMemo), not on every call.
+bool forced_rows(int* ns, int* kw) {
+  const char* v = std::getenv("EF_HIP_GEMV_ROWS");
+  return v != nullptr && std::sscanf(v, "%d,%d", ns, kw) == 2;
+}
+
+// The shape of the least estimated time for `rows` sequences (of shape (ns, kw) where ns is not 0):
+// workgroups are dealt to the CUs evenly, two to a CU at a time when their LDS allows it, plus 8 us per pair
+// for its ends.
+RowsPlan plan_rows(const GemvJob* jobs, int n_jobs, int nm, int rows, bool q8, int ns = 0, int kw = 0) {
   RowsPlan best;
   const int cus = ctx().cu_count > 0 ? ctx().cu_count : 256, nb = static_cast<int>(jobs[0].W->cols / 32);
   const size_t lim = ctx().lds_per_block > 0 ? ctx().lds_per_block : 65536;
   const int NT = (rows + kSeqTile - 1) / kSeqTile;
-  double cost = 0.0;
   for (const RowsShape& sh : kRowsShapes) {
     const size_t lds = std::max(size_t(kRowSlots) * rows_stage_bytes(sh.NS, sh.KW, !q8) + 1024,
                                 sh.KW > 1 ? static_cast<size_t>(kRowWaves) * kRowUnits * sh.NS * kWave * 16 : 0);
-    if (nb % sh.KW != 0 || lds > lim) continue;
+    if (nb % sh.KW != 0 || lds > lim || (ns != 0 && (sh.NS != ns || sh.KW != kw))) continue;
     const int groups = groups_for(jobs, n_jobs, kRowWaves / sh.KW * kRowUnits / nm * kTileRows);
     const int sgs = (NT + sh.NS - 1) / sh.NS;
     const int per_cu = (groups * sgs + cus - 1) / cus, pairs = per_cu / 2, odd = per_cu % 2;
     const double c = nb / sh.KW * (pairs * (2 * lds <= lim ? sh.t2 : 2 * sh.t1) + odd * sh.t1) + 8.0 * (pairs + odd);
-    if (best.NS != 0 && c >= cost) continue;
-    cost = c;
-    best = RowsPlan{sh.NS, sh.KW, groups, sgs, lds};
+    if (best.NS != 0 && c >= best.cost) continue;
+    best = RowsPlan{sh.NS, sh.KW, groups, sgs, lds, c};
   }
   return best;
 }
@@ -1361,25 +1376,8 @@ struct PlanMemo {
 };
 thread_local PlanMemo t_plans;
 
-// The part of plan_mfma that depends on a PlanKey only.
-Plan plan_shape(Plan p, const GemvJob* jobs, int n_jobs, int batch, size_t xld, size_t K, size_t wbytes, bool staged,
-                bool even_rt) {
-  // decided by the count of 16-sequence tiles, so workspaces sized by tile counts hold for every batch
-  const int padded = (batch + kSeqTile - 1) / kSeqTile * kSeqTile;
-  double macs = 0.0;
-  for (int j = 0; j < n_jobs; ++j) macs += static_cast<double>(jobs[j].W->rows) * p.nm * padded * K;
-  if (!staged && padded >= kRowsFrom && macs >= kRowsMacs) {
-    // A tables of every sequence tile a shape may round up to (zeros past the batch)
-    const int chunk = std::min(batch, kRowsMax), tiles = rows_tiles(chunk);
-    const size_t tab = static_cast<size_t>(tiles) * (K / 32) * 2 * kWave * 16;
-    if (tab < (size_t(1) << 32) && static_cast<size_t>(chunk) * xld * 4 < (size_t(1) << 32)) {
-      p.rows = p.ok = true;
-      p.chunk = chunk;
-      p.tab = tab;
-      p.bytes = (p.q4 ? tab : 0) + (p.q8 ? tab : 0) + static_cast<size_t>(tiles) * kSeqTile * sizeof(float);
-      return p;
-    }
-  }
+// The split-K kernel's plan for a batch (p.ok false: it has none); p holds what all plans of the launch share.
+Plan plan_split(Plan p, const GemvJob* jobs, int n_jobs, int batch, size_t K, size_t wbytes, bool even_rt) {
   p.chunk = std::min(batch, kMaxTiles * kSeqTile);
   p.NT = (p.chunk + kSeqTile - 1) / kSeqTile;
   const int nb = static_cast<int>(K / 32);
@@ -1435,6 +1433,53 @@ Plan plan_shape(Plan p, const GemvJob* jobs, int n_jobs, int batch, size_t xld, 
   return p;
 }
 
+// Estimated time of a batch's split-K GEMV and finalize kernels in us, launches after the first with the
+// preparation's fixed part: a fit to 1621 measured shapes (with the first preparation 0.89 to 1.10 of the
+// measured time for nine in ten).
+double split_us(const Plan& p, int batch, size_t K) {
+  const int cus = ctx().cu_count > 0 ? ctx().cu_count : 256;
+  const double mfma_us = static_cast<double>(p.RT) * p.nm * p.bps * 2.0 * p.NS * 16.0 / 4.0 / 2400.0;  // of a workgroup
+  double t = 0.0;
+  for (int b0 = 0; b0 < batch; b0 += p.chunk) {
+    const int nb = std::min(p.chunk, batch - b0), sg = (nb + p.NS * kSeqTile - 1) / (p.NS * kSeqTile);
+    const double part_mb = 4e-6 * p.groups * p.S * nb * p.RT * kTileRows * p.nm;
+    t += std::ceil(static_cast<double>(p.groups) * p.S * sg / cus) * (3.77 + 2.33 * mfma_us);
+    if (p.S > 1) t += 3.4 + 0.114 * part_mb;
+    if (b0 > 0) t += K <= static_cast<size_t>(kSeqPrepMaxK) ? 8.8 : 14.8;
+  }
+  return t;
+}
+
+// The part of plan_mfma that depends on a PlanKey only.
+Plan plan_shape(Plan p, const GemvJob* jobs, int n_jobs, int batch, size_t xld, size_t K, size_t wbytes, bool staged,
+                bool even_rt) {
+  // decided by the count of 16-sequence tiles, so workspaces sized by tile counts hold for every batch
+  const int padded = (batch + kSeqTile - 1) / kSeqTile * kSeqTile;
+  double macs = 0.0;
+  for (int j = 0; j < n_jobs; ++j) macs += static_cast<double>(jobs[j].W->rows) * p.nm * padded * K;
+  bool rows = !staged && padded >= kRowsFrom && macs >= kRowsMacs;
+  if (rows) {
+    const Plan sp = plan_split(p, jobs, n_jobs, padded, K, wbytes, false);
+    const RowsPlan rp = plan_rows(jobs, n_jobs, p.nm, padded, p.q8);
+    const double share = rp.KW == 1 ? 0.88 : (rp.KW == 2 ? 0.73 : 0.6);
+    rows = !sp.ok || share * rp.cost <= split_us(sp, padded, K);
+  }
+  if (forced_rows(&p.rows_ns, &p.rows_kw))
+    rows = !staged && p.rows_ns != 0 && plan_rows(jobs, n_jobs, p.nm, batch, p.q8, p.rows_ns, p.rows_kw).NS != 0;
+  if (rows) {
+    // A tables of every sequence tile a shape may round up to (zeros past the batch)
+    const int chunk = std::min(batch, kRowsMax), tiles = rows_tiles(chunk);
+    const size_t tab = static_cast<size_t>(tiles) * (K / 32) * 2 * kWave * 16;
+    if (tab < (size_t(1) << 32) && static_cast<size_t>(chunk) * xld * 4 < (size_t(1) << 32)) {
+      p.rows = p.ok = true;
+      p.chunk = chunk;
+      p.tab = tab;
+      p.bytes = (p.q4 ? tab : 0) + (p.q8 ? tab : 0) + static_cast<size_t>(tiles) * kSeqTile * sizeof(float);
+      return p;
+    }
+  }
+  return plan_split(p, jobs, n_jobs, batch, K, wbytes, even_rt);
+}
 
 // staged: the launch reads producer-staged tables (never the many-sequence kernel); even_rt: only shapes
 // whose workgroup rows are a multiple of 32 (outputs staged as tables).
@@ -1620,7 +1665,8 @@ int launch_gemv_mfma(const GemvJob* jobs, int n_jobs, int epi, const float* norm
     p.t8 = t8;
     p.post = post;
     const int nbk = static_cast<int>(K / 32);
-    const RowsPlan rp = pl.rows ? plan_rows(jobs, n_jobs, pl.nm, nb, pl.q8) : RowsPlan{};
+    const RowsPlan rp =
+        pl.rows ? plan_rows(jobs, n_jobs, pl.nm, nb, pl.q8, pl.rows_ns, pl.rows_kw) : RowsPlan{};
     const int rows_wg = pl.rows ? kRowWaves / rp.KW * kRowUnits / pl.nm * kTileRows : pl.RT * kTileRows;
     const int prep_tiles = pl.rows ? rp.sgs * rp.NS : pl.SG * pl.NS;  // tiles past B get zeros
     if (K <= static_cast<size_t>(kSeqPrepMaxK)) {
