@@ -10,6 +10,7 @@ at B = 64) and mixed-type launches; epilogues and the fused RMSNorm are checked 
 import os
 import subprocess
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -261,10 +262,64 @@ def test_many_sequence_kernel_swiglu_and_mixed_jobs(hip):
         assert err.max() < REL_TOL
 
 
+def _in_new_thread(f):
+    """f() in a thread of its own, which plans its launches anew (EF_HIP_GEMV_ROWS is read there)."""
+    box = []
+
+    def run():
+        try:
+            box.append((f(), None))
+        except BaseException as e:  # re-raised below
+            box.append((None, e))
+
+    t = threading.Thread(target=run)
+    t.start()
+    t.join()
+    if box[0][1] is not None:
+        raise box[0][1]
+    return box[0][0]
+
+
+@pytest.mark.parametrize("stages", [1, 3, 17])  # a single one, an odd count, two flushes and one stage more
+@pytest.mark.parametrize("qtype,ns,kw", [(qt, *s) for s in ((4, 1), (3, 1), (4, 2), (3, 2), (2, 2), (4, 4), (2, 4))
+                                         for qt in (O.Q4_0, O.Q8_0)
+                                         if (qt, *s) != (O.Q8_0, 4, 4)])  # whose stages do not fit the LDS
+def test_many_sequence_kernel_every_shape(hip, monkeypatch, qtype, ns, kw, stages):
+    """Each instantiated shape of the many-sequence kernel (ns sequence tiles, kw K shares), forced by
+    EF_HIP_GEMV_ROWS: a partial row tile and workgroup (150 rows), a partial sequence tile and group, and more
+    than 8 sequence groups (600 sequences); store and residual of one matrix, SwiGLU of two."""
+    rows, K = 150, 32 * kw * stages
+    print(f"[case] many-sequence kernel ns={ns} kw={kw} qtype={qtype} K={K}", flush=True)
+    monkeypatch.setenv("EF_HIP_GEMV_ROWS", f"{ns},{kw}")
+    pk = [D.random_rows(qtype, rows, K, seed=150 + K + i) for i in range(2)]
+    w64 = [D.dequant_exact(qtype, p, K) for p in pk]
+    G, U = [hip.Weight(qtype, rows, K, host=p) for p in pk]
+    for batch in (35, 600):
+        X = (D.rng(batch).standard_normal((batch, K)) * np.exp(D.rng(K).normal(size=(batch, 1)))).astype(np.float32)
+        base = D.rng(3).standard_normal((batch, rows)).astype(np.float32)
+        dx, ds, dr, dg = hip.DeviceArray.from_host(X), *[hip.DeviceArray.from_host(base) for _ in range(3)]
+
+        def calls():
+            hip.matvec(G, dx, ds, batch=batch)
+            hip.matvec_residual(G, dx, dr, batch=batch)
+            hip.matvec_swiglu(G, U, dx, dg, batch=batch)
+
+        _in_new_thread(calls)
+        got = ds.numpy()
+        _exact_close(w64[0], X, got, "store")
+        assert np.abs(dr.numpy() - (base + got)).max() <= 2.0 ** -23 * (np.abs(base) + np.abs(got)).max()
+        x = X.astype(np.float64)
+        g, u = [x @ w.T for w in w64]
+        sg, su = [np.abs(x) @ np.abs(w).T for w in w64]
+        with np.errstate(over="ignore"):
+            want = g / (1 + np.exp(-g)) * u
+        bound = 1e-5 * (1.1 * sg * np.abs(u) + np.abs(g) * su) + 1e-6 * np.abs(want) + 1e-10 * sg * su  # as above
+        assert (np.abs(dg.numpy() - want) <= bound).all()
+
+
 def test_kept_workspace_is_shared_in_order(hip):
     """Calls on the library's stream keep one workspace: calls of different shapes in turn and from two
     threads give the bits of calls on a stream of their own (which allocate)."""
-    import threading
     shapes = [(128, 1024, 5), (64, 2048, 40), (256, 5632, 64), (96, 4096, 300), (128, 1024, 5)]
     work = []
     for i, (rows, cols, batch) in enumerate(shapes):
