@@ -505,31 +505,20 @@ int ensure_prefill(ef_hip_engine e, size_t rows) {
     const GemvJob o{w.wo, nullptr, bufs[4], bufs[0], c.D, c.D};
     const GemvJob gu{w.w_gate, w.w_up, bufs[0], bufs[5], c.D, c.F};
     const GemvJob dn{w.w_down, nullptr, bufs[5], bufs[0], c.F, c.D};
-    // the workspace depends on the shapes and types only: a layer like the one before needs no more
-    if (l > 0) {
-      const ef_hip_layer& v = e->layers[l - 1];
-      if (w.wq->qtype == v.wq->qtype && w.wk->qtype == v.wk->qtype && w.wv->qtype == v.wv->qtype &&
-          w.wo->qtype == v.wo->qtype && w.w_gate->qtype == v.w_gate->qtype && w.w_down->qtype == v.w_down->qtype)
-        continue;
-    }
-    // every row count a launch may use (a last chunk is shorter): row counts up to 128 one by one, then
-    // every multiple of a 16-row tile up to 1024 (the split-K kernel's largest launch; within a tile
-    // count the workspace grows with the rows), and the full count (the many-sequence kernel's grows
-    // with the rows)
-    const int cap = static_cast<int>(std::min<size_t>(rows, 1024));
-    std::vector<int> counts;
-    for (int r = 2; r <= std::min(cap, 128); ++r) counts.push_back(r);
-    for (int r = 144; r <= cap; r += 16) counts.push_back(r);
-    counts.push_back(cap);
-    counts.push_back(static_cast<int>(rows));
-    for (const int r : counts) {
-      const GemvJob lm{e->lm_head, nullptr, bufs[0], nullptr, c.D, c.V};
-      need = std::max({need, gemv_mfma_workspace_bytes(qkv, 3, kEpiStore, r, c.D),
-                       gemv_mfma_workspace_bytes(&o, 1, kEpiResidual, r, c.D),
-                       gemv_mfma_workspace_bytes(&gu, 1, kEpiSwiglu, r, c.D),
-                       gemv_mfma_workspace_bytes(&dn, 1, kEpiResidual, r, c.F),
-                       gemv_mfma_workspace_bytes(&lm, 1, kEpiStore, r, c.D)});
-    }
+    const GemvJob lm{e->lm_head, nullptr, bufs[0], nullptr, c.D, c.V};
+    // for every row count a launch may use (a last chunk is shorter); it depends on the shapes and types only: a
+    // product like the one of the layer before needs no more
+    const ef_hip_layer* v = l > 0 ? &e->layers[l - 1] : nullptr;
+    const int r = static_cast<int>(rows);
+    if (v == nullptr || w.wq->qtype != v->wq->qtype || w.wk->qtype != v->wk->qtype || w.wv->qtype != v->wv->qtype)
+      need = std::max(need, gemv_mfma_workspace_upto(qkv, 3, kEpiStore, r, c.D));
+    if (v == nullptr || w.wo->qtype != v->wo->qtype)
+      need = std::max(need, gemv_mfma_workspace_upto(&o, 1, kEpiResidual, r, c.D));
+    if (v == nullptr || w.w_gate->qtype != v->w_gate->qtype)
+      need = std::max(need, gemv_mfma_workspace_upto(&gu, 1, kEpiSwiglu, r, c.D));
+    if (v == nullptr || w.w_down->qtype != v->w_down->qtype)
+      need = std::max(need, gemv_mfma_workspace_upto(&dn, 1, kEpiResidual, r, c.F));
+    if (v == nullptr) need = std::max(need, gemv_mfma_workspace_upto(&lm, 1, kEpiStore, r, c.D));
   }
   void* ws = nullptr;
   if (need > 0 && hipMalloc(&ws, need) != hipSuccess) {

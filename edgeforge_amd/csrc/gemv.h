@@ -27,6 +27,8 @@ struct GemvJob {
 // for the same launch) holds the prepared activation fragments and the split-K partial sums;
 // without it the launch allocates stream-ordered memory.  0 when the launch does not take this path.
 size_t gemv_mfma_workspace_bytes(const GemvJob* jobs, int n_jobs, int epi, int batch, size_t ldx);
+// A workspace for every such launch of at most `rows` sequences (a prefill's chunks).
+size_t gemv_mfma_workspace_upto(const GemvJob* jobs, int n_jobs, int epi, int rows, size_t ldx);
 // The batched path reads Q4_0 / Q8_0 matrices from a tile-order copy (w->tiled, tiled_bytes(w)
 // bytes).  ensure_tiled makes it when missing (allocates; refused while `s` is capturing a graph).
 // refresh_tiled rewrites an existing copy from the handle's current bytes, in place and

@@ -1240,6 +1240,7 @@ struct Plan {
   bool q4 = false, q8 = false;
   int nm = 1, NT = 1, RT = 2, NS = 1, SG = 1, groups = 0, S = 1, bps = 0, chunk = 0;
   size_t tab = 0, part_off = 0, bytes = 0, lds = 0;
+  size_t most = 0;  // the larger of what this kernel and the one not chosen need
   double cost = 0.0;
   bool rows = false;  // the many-sequence kernel (plan_rows per launch)
   int rows_ns = 0, rows_kw = 0;  // its shape, where EF_HIP_GEMV_ROWS names one
@@ -1457,28 +1458,33 @@ Plan plan_shape(Plan p, const GemvJob* jobs, int n_jobs, int batch, size_t xld, 
   const int padded = (batch + kSeqTile - 1) / kSeqTile * kSeqTile;
   double macs = 0.0;
   for (int j = 0; j < n_jobs; ++j) macs += static_cast<double>(jobs[j].W->rows) * p.nm * padded * K;
-  bool rows = !staged && padded >= kRowsFrom && macs >= kRowsMacs;
-  if (rows) {
-    const Plan sp = plan_split(p, jobs, n_jobs, padded, K, wbytes, false);
-    const RowsPlan rp = plan_rows(jobs, n_jobs, p.nm, padded, p.q8);
-    const double share = rp.KW == 1 ? 0.88 : (rp.KW == 2 ? 0.73 : 0.6);
-    rows = !sp.ok || share * rp.cost <= split_us(sp, padded, K);
-  }
-  if (forced_rows(&p.rows_ns, &p.rows_kw))
-    rows = !staged && p.rows_ns != 0 && plan_rows(jobs, n_jobs, p.nm, batch, p.q8, p.rows_ns, p.rows_kw).NS != 0;
-  if (rows) {
+  int ns = 0, kw = 0;
+  const bool forced = forced_rows(&ns, &kw);
+  if (!staged && (forced ? ns != 0 : padded >= kRowsFrom && macs >= kRowsMacs)) {
     // A tables of every sequence tile a shape may round up to (zeros past the batch)
     const int chunk = std::min(batch, kRowsMax), tiles = rows_tiles(chunk);
     const size_t tab = static_cast<size_t>(tiles) * (K / 32) * 2 * kWave * 16;
-    if (tab < (size_t(1) << 32) && static_cast<size_t>(chunk) * xld * 4 < (size_t(1) << 32)) {
-      p.rows = p.ok = true;
-      p.chunk = chunk;
-      p.tab = tab;
-      p.bytes = (p.q4 ? tab : 0) + (p.q8 ? tab : 0) + static_cast<size_t>(tiles) * kSeqTile * sizeof(float);
-      return p;
+    const RowsPlan rp = plan_rows(jobs, n_jobs, p.nm, padded, p.q8, ns, kw);
+    if (rp.NS != 0 && tab < (size_t(1) << 32) && static_cast<size_t>(chunk) * xld * 4 < (size_t(1) << 32)) {
+      const Plan sp = plan_split(p, jobs, n_jobs, padded, K, wbytes, false);
+      const double share = rp.KW == 1 ? 0.88 : (rp.KW == 2 ? 0.73 : 0.6);
+      const bool rows = forced || !sp.ok || share * rp.cost <= split_us(sp, padded, K);
+      Plan r = p;
+      r.rows = r.ok = true;
+      r.rows_ns = ns;
+      r.rows_kw = kw;
+      r.chunk = chunk;
+      r.tab = tab;
+      r.bytes = (p.q4 ? tab : 0) + (p.q8 ? tab : 0) + static_cast<size_t>(tiles) * kSeqTile * sizeof(float);
+      const size_t most = std::max(r.bytes, sp.ok ? sp.bytes : 0);
+      if (!rows) r = batch == padded ? sp : plan_split(p, jobs, n_jobs, batch, K, wbytes, even_rt);
+      r.most = std::max(r.bytes, most);
+      return r;
     }
   }
-  return plan_split(p, jobs, n_jobs, batch, K, wbytes, even_rt);
+  p = plan_split(p, jobs, n_jobs, batch, K, wbytes, even_rt);
+  p.most = p.bytes;
+  return p;
 }
 
 // staged: the launch reads producer-staged tables (never the many-sequence kernel); even_rt: only shapes
@@ -1570,6 +1576,23 @@ size_t gemv_mfma_workspace_bytes(const GemvJob* jobs, int n_jobs, int epi, int b
   return p.ok ? p.bytes : 0;
 }
 
+size_t gemv_mfma_workspace_upto(const GemvJob* jobs, int n_jobs, int epi, int rows, size_t ldx) {
+  // Row counts up to 128 one by one, then every multiple of a 16-row tile up to the split-K kernel's largest
+  // launch (launch_gemv_mfma: a count between takes its tile's plan if its own wants more), and the full count,
+  // with what the kernel not chosen there needs too: past that launch the split-K kernel's need stays and the
+  // many-sequence kernel's grows with the rows, and either may be chosen at a count between.
+  const int cap = std::min(rows, kMaxTiles * kSeqTile);
+  size_t need = 0;
+  auto at = [&](int r) {
+    const Plan p = plan_mfma(jobs, n_jobs, epi, r, ldx);
+    if (p.ok) need = std::max(need, p.most);
+  };
+  for (int r = 2; r <= std::min(cap, 128); ++r) at(r);
+  for (int r = 144; r <= cap; r += kSeqTile) at(r);
+  at(cap);
+  at(rows);
+  return need;
+}
 
 namespace {
 // The workspace of calls on the library's own stream that bring none: kept from call to call (a
@@ -1617,8 +1640,14 @@ int release_gemv_workspace(hipStream_t stream) {
 int launch_gemv_mfma(const GemvJob* jobs, int n_jobs, int epi, const float* norm_w, float eps, int batch, size_t ldx,
                      size_t ldy, void* ws, size_t ws_bytes, hipStream_t stream, bool* taken) {
   *taken = false;
-  const Plan pl = plan_mfma(jobs, n_jobs, epi, batch, ldx);
+  Plan pl = plan_mfma(jobs, n_jobs, epi, batch, ldx);
   if (!pl.ok) return EF_HIP_OK;
+  if (ws != nullptr && ws_bytes < pl.bytes) {
+    // within a tile count the cheapest split of K may change with the batch, and its workspace with it: a
+    // workspace sized by tile counts holds the plan of the whole tiles
+    const Plan whole = plan_mfma(jobs, n_jobs, epi, (batch + kSeqTile - 1) / kSeqTile * kSeqTile, ldx);
+    if (whole.ok && whole.bytes <= ws_bytes) pl = whole;
+  }
   if (norm_w != nullptr && reinterpret_cast<uintptr_t>(norm_w) % 16 != 0) return EF_HIP_OK;
   for (int j = 0; j < n_jobs; ++j) {
     EFH_RC(ensure_tiled(jobs[j].W, stream));
