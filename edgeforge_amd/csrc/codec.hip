@@ -84,12 +84,16 @@ __device__ float q4_scale(const float (&x)[32], bool search) {
     }
   }
   if (!(amax > 0.0f) || !isfinite(amax)) return 0.0f;
+  if (!search) {  // one candidate: its error decides nothing
+    const float d = fp16_round(fminf(fmaxf(__fdiv_rn(smax, -8.0f), -65504.0f), 65504.0f));
+    return d != 0.0f ? d : 0.0f;
+  }
   // at |d| >= 2^-24, the least fp16 scale, |x / d| <= amax 2^24
   const bool clean = __all(!nan && amax < 64.0f);
   auto sse_of = [&](float d) { return clean ? q4_sse<true>(x, d) : q4_sse<false>(x, d); };
   float best = 0.0f;
   double best_sse = -1.0;
-  for (int c = 0; c < (search ? 6 : 1); ++c) {
+  for (int c = 0; c < 6; ++c) {
     const float num = c == 0 ? smax : amax;
     const float den = c == 0 ? -8.0f : (c == 5 ? 8.0f : 6.75f + 0.25f * static_cast<float>(c));  // 7, 7.25, 7.5, 7.75, 8
     const float d = fp16_round(fminf(fmaxf(__fdiv_rn(num, den), -65504.0f), 65504.0f));
@@ -101,7 +105,6 @@ __device__ float q4_scale(const float (&x)[32], bool search) {
     }
   }
   if (best_sse < 0.0) return 0.0f;
-  if (!search) return best;
   for (int round = 0; round < 2; ++round) {
     // least squares over the codes of the best scale: integer products and their sum are exact
     const float inv = __fdiv_rn(1.0f, best);
@@ -132,7 +135,7 @@ __device__ float q4_scale(const float (&x)[32], bool search) {
 // same way.  Bound by vector issue: eight tries of 32 weights at seven instructions, four of them on
 // doubles (the reference's sequential double sums).  Q4_0 with the search, 5632x2048: 54.5 us per call
 // with strided loads, codes kept per try and twice the instructions, 39.8 us so (1.3 TB/s; 500x512
-// 14.5 -> 10.5); Q8_0 11.7 -> 10.9 (4.8 TB/s).  256 blocks per workgroup cost small matrices 0.7 to 2 us.
+// 14.5 -> 10.5), without it 15.9 -> 12.8; Q8_0 11.7 -> 10.9 (5.4 TB/s).  256 blocks per workgroup cost small matrices 0.7 to 2 us.
 constexpr int kQuantBlocks = 64;  // one wave: small matrices reach more CUs, and the tail is short
 
 template <bool Q4>
@@ -143,20 +146,29 @@ __global__ __launch_bounds__(kQuantBlocks) void quantize_blocks_kernel(const flo
   const long g0 = static_cast<long>(blockIdx.x) * kQuantBlocks;
   const int n = static_cast<int>(min(static_cast<long>(kQuantBlocks), blocks - g0)), t = threadIdx.x;
   const float* src = w + g0 * 32;
-  if (n == kQuantBlocks && reinterpret_cast<uintptr_t>(src) % 16 == 0) {
+  const bool aligned = reinterpret_cast<uintptr_t>(src) % 16 == 0;
+  auto put4 = [&](int q, float4 v) {  // the workgroup's weights 4 q .. 4 q + 3
+    float* p = xs + (q >> 3) * kLd + 4 * (q & 7);
+    p[0] = v.x;
+    p[1] = v.y;
+    p[2] = v.z;
+    p[3] = v.w;
+  };
+  if (n == kQuantBlocks && aligned) {
     float4 v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = reinterpret_cast<const float4*>(src)[t + kQuantBlocks * i];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = 4 * (t + kQuantBlocks * i);
-      float* p = xs + (e >> 5) * kLd + (e & 31);
-      p[0] = v[i].x;
-      p[1] = v[i].y;
-      p[2] = v[i].z;
-      p[3] = v[i].w;
-    }
-  } else {  // the last blocks, or weights off a 16-byte boundary
+    for (int i = 0; i < 8; ++i) put4(t + kQuantBlocks * i, v[i]);
+  } else if (aligned) {  // the last blocks
+    float4 v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      v[i] = t + kQuantBlocks * i < n * 8 ? reinterpret_cast<const float4*>(src)[t + kQuantBlocks * i]
+                                          : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) put4(t + kQuantBlocks * i, v[i]);
+  } else {  // weights off a 16-byte boundary
     float v[32];
 #pragma unroll
     for (int i = 0; i < 32; ++i) v[i] = t + kQuantBlocks * i < n * 32 ? src[t + kQuantBlocks * i] : 0.0f;

@@ -208,26 +208,28 @@ def test_rows_f32_is_exact_dequantization(hip, qtype):
         assert np.array_equal(got[i].view(np.uint32), ref[r].view(np.uint32))
 
 
-@pytest.mark.parametrize("qtype", [O.Q4_0, O.Q8_0])
+@pytest.mark.parametrize("qtype,search", [(O.Q4_0, 1), (O.Q4_0, 0), (O.Q8_0, 1)])
 @pytest.mark.parametrize("rows,cols,off", [(1, 32, 0), (3, 96, 0), (63, 32, 0), (65, 32, 0), (257, 32, 0), (5, 4128, 1)])
-def test_quantizer_block_counts_and_alignment(hip, qtype, rows, cols, off):
+def test_quantizer_block_counts_and_alignment(hip, qtype, search, rows, cols, off):
     """Block counts around the workgroups (one, partial, one more) and, with off, an input at a 4-byte
     and an output at an odd address: bytes identical to the oracle, and none written past the end.
-    Weights of every size the clamp meets: values whose codes overflow an int next to NaN blocks."""
-    print(f"[case] quantizer qtype={qtype} {rows}x{cols} off={off}", flush=True)
+    Weights of every size the clamp meets: values whose codes overflow an int next to NaN blocks, and blocks
+    whose scale underflows to a zero of either sign."""
+    print(f"[case] quantizer qtype={qtype} search={search} {rows}x{cols} off={off}", flush=True)
     g = D.rng(rows * cols + off)
     w = (g.standard_normal((rows, cols)) * np.exp(g.normal(0, 6, (rows, cols // 32)).repeat(32, 1))).astype(np.float32)
     w[0, 3] = np.nan
+    w[rows // 2:rows // 2 + 2, :32] = g.uniform(-1e-8, 1e-8, (w[rows // 2:rows // 2 + 2].shape[0], 32))
     w[-1, 31] = 3e38
     dw = hip.DeviceArray((rows * cols + off,))
     dw.upload(np.concatenate([np.zeros(off, np.float32), w.reshape(-1)]))
     nb = rows * O.row_bytes(qtype, cols)
     out = hip.DeviceArray((nb + off + 64,), np.uint8)
     out.upload(np.full(nb + off + 64, 0xA5, np.uint8))
-    L.call("ef_hip_quantize", qtype, dw.at(off), rows, cols, 1, out.at(off), None)
+    L.call("ef_hip_quantize", qtype, dw.at(off), rows, cols, search, out.at(off), None)
     got = out.numpy()
     want = np.empty((rows, O.row_bytes(qtype, cols)), np.uint8)
     for r in range(rows):
-        assert O.lib().efo_quantize_row(qtype, O.ptr(w[r], O._f32p), cols, O.ptr(want[r], O._u8p), 1) == 0
+        assert O.lib().efo_quantize_row(qtype, O.ptr(w[r], O._f32p), cols, O.ptr(want[r], O._u8p), search) == 0
     assert np.array_equal(got[off:off + nb], want.reshape(-1))
     assert (got[:off] == 0xA5).all() and (got[off + nb:] == 0xA5).all()
