@@ -135,7 +135,8 @@ __device__ float q4_scale(const float (&x)[32], bool search) {
 // same way.  Bound by vector issue: eight tries of 32 weights at seven instructions, four of them on
 // doubles (the reference's sequential double sums).  Q4_0 with the search, 5632x2048: 54.5 us per call
 // with strided loads, codes kept per try and twice the instructions, 39.8 us so (1.3 TB/s; 500x512
-// 14.5 -> 10.5), without it 15.9 -> 12.8; Q8_0 11.7 -> 10.9 (5.4 TB/s).  256 blocks per workgroup cost small matrices 0.7 to 2 us.
+// 14.5 -> 10.5), without it 15.9 -> 12.8; Q8_0 11.7 -> 10.9 (5.4 TB/s).  256 blocks per workgroup cost small
+// matrices 0.7 to 2 us.
 constexpr int kQuantBlocks = 64;  // one wave: small matrices reach more CUs, and the tail is short
 
 template <bool Q4>

@@ -59,7 +59,7 @@ constexpr int kTP = 1024;                       // prep workgroup
 constexpr int kWavesP = kTP / kWave;
 constexpr int kTileRows = 16;
 constexpr int kSeqTile = 16;                    // sequences per A operand (one per row)
-constexpr int kMaxTiles = 64;                   // sequence tiles per launch: 1024 sequences (rows)
+constexpr int kMaxTiles = 64;                   // sequence tiles per split-K launch: 1024 sequences (rows)
 constexpr int kMaxJobsM = 4;
 constexpr int kPrepBlocks = kTP / kWave;        // blocks per xfrag workgroup: one per wave
 // K blocks per wave of one batched GEMV workgroup: 24 for the smallest shapes (two accumulator
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(kTP) void xfrag_kernel(PrepArgs a) {
   //     column orders (Q4_0: weights 4g..4g+3 and 4g+16..4g+19 of the block, Q8_0: 8g..8g+7)
   const int kb = blockIdx.x * kPrepBlocks + wave;
   const int i = lane & 15, g = lane >> 4, sq_f = tile * kSeqTile + i;
-  // one resource over the chunk's rows (B * ldx floats, < 16 MiB); a lane of a sequence past the
+  // one resource over the chunk's rows (B * ldx floats, below 4 GiB: plan_shape); a lane of a sequence past the
   // batch, or of a block past K, addresses the resource's end and reads zeros
   const uint32_t x_bytes = static_cast<uint32_t>(a.B) * static_cast<uint32_t>(a.ldx) * 4u;
   const __amdgpu_buffer_rsrc_t rx_all = make_rsrc(a.x, x_bytes);

@@ -22,7 +22,7 @@ struct AttnArgs {
   float scale;          // float(1 / sqrt(hd))
   int pre_vrows;        // set by launch_attention: the first chunk's V rows have their own LDS
   int chunk;            // set by launch_attention: rows of the LDS staging buffer (>= 64)
-  AEmit em;             // KV-group kernel: ctx also staged as the o-projection's tables (afrag.h)
+  AEmit em;             // KV-group and large-batch kernels: ctx also staged as the o-projection's tables (afrag.h)
   // Position-split decode (attention_split_kernel, then attention_combine_kernel): `splits`
   // workgroups per (sequence, KV group), each over `span` positions; part holds their partial
   // results.  part == nullptr: no split.
@@ -53,7 +53,8 @@ size_t attention_lds_bytes(int hd, int max_seq);
 // 2048 positions at 8 heads per KV head).  part_floats: the workspace it needs.
 bool attention_split_plan(int H, int KV, int hd, int max_seq, int batch, int* splits, int* span, size_t* part_floats);
 int launch_attention(const AttnArgs& a, int batch, hipStream_t s);
-// Whether launch_attention runs the KV-group kernel (the one that can stage ctx as tables).
+// Whether launch_attention runs the KV-group kernel or, in its place, the large-batch one (the two that can stage
+// ctx as tables).
 bool attention_uses_group(const AttnArgs& a, int batch);
 int launch_rmsnorm(const float* x, const float* w, float eps, int n, long ld, int batch, float* out, hipStream_t s);
 // With out_eos: eos_p[b] is stored beside the picked token (the chat loop's per-step P(EOS)).

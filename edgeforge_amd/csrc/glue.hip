@@ -3,10 +3,12 @@
 // final RMSNorm output, and the bookkeeping that feeds a picked token back as the next input.
 // Positions and token ids are read from device memory so one captured HIP graph serves every step.
 //
-// Arithmetic follows the reference's operation order with contraction off: the per-position dot
+// The vector kernels follow the reference's operation order with contraction off: the per-position dot
 // product uses the 8-way partial sums of kern::dot_f32 (src/kernels.cpp:27-43), softmax subtracts
 // the max, uses float exp and a double sum (:77-92), and each output dimension accumulates p * v
-// over positions in order (:168-172).
+// over positions in order (:168-172).  The two matrix-core kernels, the defaults at hd = 64 for large batches
+// (attention_batch_kernel) and for prompts but the shortest (prefill_mfma_kernel), do not: scores in four
+// partial sums, exponentials of base 2 against a running maximum, p * v summed by chunks.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -1265,8 +1267,8 @@ constexpr int kPfPairs = 64, kPfChunk = 64, kPfLd = 68;
 // over 32 KV heads, one position of one sequence (32 workgroups of one pair) 69 / 71 from position 0,
 // 96 / 93 from 500, 211 / 175 from 2000, 714 / 492 from 8000; two positions of 32 sequences (1024 of two) 108 / 109
 // from 0, 205 / 170 from 500.  Only workgroups of a single pair that do not fit the CUs at once are
-// left to the rows kernel: one position of 32 sequences (1024) 89 / 94 from 0, 147 / 154 from 500, of 16 (512) 85 / 87 and
-// 128 / 118.
+// left to the rows kernel: one position of 32 sequences (1024) 89 / 94 from 0, 147 / 154 from 500, of 16 (512)
+// 85 / 87 and 128 / 118.
 constexpr int kPfMfmaFrom = 128, kPfMfmaWorkgroups = 32;
 
 __global__ __launch_bounds__(256, 3) void prefill_mfma_kernel(PrefillArgs pa, int nseq, int cus) {

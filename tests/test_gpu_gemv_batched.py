@@ -1,6 +1,6 @@
 """GPU parity of the batched (2+ sequences) packed GEMV on the matrix cores (C-ABI calls).
 
-Every sequence of a batch must meet the single-vector gates (BASELINE.json north_star):
+Every sequence of a batch must meet the single-vector gates:
 |gpu - exact| <= 1e-5 * sum|w x| per row (tests/test_qinfer.cpp:95) and max |gpu - cpu fp32| <= 1e-4
 against the oracle's AVX2 kernel (src/qkernels.cpp:131-180) on that sequence alone.  Shapes cover
 batches that are not a multiple of the 16-sequence tile, many tiles in one launch, more than 1024
@@ -39,11 +39,11 @@ def _batch_x(seed, batch, cols):
     (O.Q4_0, 96, 512, 300),      # 19 sequence tiles in one launch
     (O.Q8_0, 37, 256, 1100),     # two launches (1024 + 76 sequences)
     (O.Q8_0, 64, 512, 2),
-    (O.Q4_0, 5632, 2048, 16),    # config 4 at B = 16: gate / up shape
+    (O.Q4_0, 5632, 2048, 16),    # TinyLlama gate / up shape at B = 16
     (O.Q4_0, 2048, 5632, 16),    # down shape (K = 5632)
     (O.Q8_0, 256, 2048, 16),     # a Q8_0 k / v override
     (O.Q4_0, 2048, 2048, 16),    # q / o shape
-    (O.Q4_0, 5632, 2048, 64),    # config 4 at B = 64
+    (O.Q4_0, 5632, 2048, 64),    # the same at B = 64
     (O.Q8_0, 256, 2048, 64),
 ])
 def test_batched_gemv_each_sequence_meets_the_gates(hip, qtype, rows, cols, batch):

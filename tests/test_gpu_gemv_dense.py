@@ -2,8 +2,8 @@
 
 kern::matvec_rows dispatches all five storage types (src/qkernels.cpp:213-269); these three reach
 the decode path through lossless .efq files, tied embeddings and the quantizer's BF16 fallback for
-row lengths that are not a multiple of 32.  Gates as for the packed types (BASELINE.json
-north_star, tests/test_qinfer.cpp:95): |gpu - exact| <= 1e-5 * sum|w x| per row against a float64
+row lengths that are not a multiple of 32.  Gates as for the packed types
+(tests/test_qinfer.cpp:95): |gpu - exact| <= 1e-5 * sum|w x| per row against a float64
 dot of the exactly decoded weights, and max |gpu - cpu| <= 1e-4 against the oracle's AVX2 kernels
 (dot_bf16_avx2 / dot_f32_avx2 / the F16 loop, src/qkernels.cpp:182-234).  Shapes cover the 16-byte
 vector path, odd row lengths (per-element path), a partial last tile, batches and every epilogue.
